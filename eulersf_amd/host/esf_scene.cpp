@@ -433,7 +433,8 @@ extern "C" esf_status esf_scene_load_cfg(const char* path, int precision, esf_ct
   }
   // smoke carpet  main.cpp:80-90
   const double carpet = cfg.getFloat("smoke carpet thickness", 0.06);
-  const int layers = (int)(carpet / g.dh);
+  // (a carpet thicker than the box ends at its top)
+  const int layers = (int)std::min(carpet / g.dh, (double)g.yres);
   const size_t N = (size_t)g.xres * g.yres * g.zres;
   std::vector<double> inten(N, 0.0);
   for (int z = 1; z < g.zres - 1; z++)
