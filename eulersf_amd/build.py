@@ -30,6 +30,7 @@ FLAGS = [
 ]
 SOURCES = [
     os.path.join(CSRC, "esf_pressure.hip"),
+    os.path.join(CSRC, "esf_fastdiag.hip"),
     os.path.join(CSRC, "esf_solid.hip"),
     os.path.join(CSRC, "esf_grid.hip"),
     os.path.join(CSRC, "esf_mesh.hip"),

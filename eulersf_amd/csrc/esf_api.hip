@@ -7,6 +7,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "esf_fastdiag.h"
 #include "esf_internal.h"
 
 namespace esf {
@@ -23,7 +24,6 @@ esf_status crSolve(esf_ctx* ctx, int which, const T* minv, const T* b, const T* 
 esf_status mixedSolve(esf_ctx* ctx, double eps, int maxIt, int* iters, bool* converged,
                       double* relres, int* refinements, int* innerIters,
                       bool scalarsReady = false);
-int spmvBlocks(const esf_ctx* ctx);
 void spmvConfigure(esf_ctx* ctx);
 esf_status benchPressureApply(esf_ctx* ctx, int fp32, int reps, double* avgMs);
 esf_status benchCopy(esf_ctx* ctx, long bytes, int reps, double* avgMs);
@@ -269,6 +269,7 @@ esf_status esf_ctx_create(esf_ctx** out, const esf_grid* g, const esf_params* p)
   spmvConfigure(ctx);
   ctx->nPartials = std::max<int>(5 * std::max(spmvBlocks(ctx), cdiv(N, 128)) + 64, 1 << 16);
   if (!st) st = dalloc(ctx, &ctx->partials, ctx->nPartials);
+  if (!st && mixed && fdFits(d)) st = fdCreate(ctx);
   if (!st) st = dalloc(ctx, &ctx->energyPart, cdiv(N, 256));
   if (!st) st = dalloc(ctx, &ctx->sc, 8);
   if (!st) st = dalloc(ctx, &ctx->dmisc, 16);

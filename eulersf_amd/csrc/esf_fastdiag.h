@@ -1,0 +1,66 @@
+// esf_fastdiag.h -- the pieces of the fast-diagonalisation preconditioned
+// pressure solve shared by esf_fastdiag.hip (the preconditioner and the
+// vector update) and esf_pressure.hip (the SpMV and the solve).
+#pragma once
+#include "esf_internal.h"
+
+namespace esf {
+
+// cells per axis, padded to multiples of 16, and the 32-wide tiles of x and y
+struct FdGeom {
+  int nx, ny, nz, PX, PY, PZ, tx, ty;
+};
+
+// the test of the recursive residual that an iteration's first kernel makes
+struct PcgTest {
+  int nb;               // |r|^2 partials of the update before
+  const double* parts;
+  double tol2;          // (relative tolerance)^2
+  int iter;             // updates made so far
+  CrScalars* sc;        // the solve's block
+  const CrScalars* outer;  // holds |b|
+};
+
+// what the SpMV needs to form p = z + beta p: the r . z partials, and r . z of
+// this and the last iteration at rz[iter & 1], rz[1 - (iter & 1)]
+struct PcgDir {
+  int iter;
+  int nb;
+  const double* parts;
+  double* rz;
+};
+
+// the sum of nb partials, in every thread of the block (256 threads) and
+// bitwise the same in every block; lds: 4 doubles
+__device__ inline double blockTotal(int nb, const double* __restrict__ parts, double* lds) {
+  double a[4] = {0, 0, 0, 0};
+  for (int i = threadIdx.x; i < nb; i += 4 * 256) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) a[u] += i + 256 * u < nb ? parts[i + 256 * u] : 0.0;
+  }
+  const double w = waveSum((a[0] + a[1]) + (a[2] + a[3]));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
+  __syncthreads();
+  const double s = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+  __syncthreads();
+  return s;
+}
+
+FdGeom fdGeom(const Dims& d);
+// whether the preconditioner takes this grid
+bool fdFits(const Dims& d);
+// its tables and buffers (mixed contexts, at creation)
+esf_status fdCreate(esf_ctx* ctx);
+// one iteration: z = S0^-1 r, p = z + beta p, q = S p, x += alpha p,
+// r -= alpha q; on scalar block 1, |b| in block 0
+esf_status fdIteration(esf_ctx* ctx, int it, double eps);
+// the test of the residual after `it` iterations; scalar block 1 to hostOut
+void fdTest(esf_ctx* ctx, int it, double eps, CrScalars* hostOut);
+
+// esf_pressure.hip
+int spmvBlocks(const esf_ctx* ctx);
+esf_status spmvPcg(esf_ctx* ctx, const double* pOld, const float* z, double* pNew, double* q,
+                   CrScalars* sc, const PcgDir& dir, double* parts);
+
+}  // namespace esf

@@ -1,0 +1,524 @@
+// esf_fastdiag.hip -- the mixed form's pressure solve: conjugate gradients in
+// FP64 on S x = b, S = J M^-1 J^T, preconditioned by the inverse of the same
+// operator with one mass at every interior node, applied in FP32 by fast
+// diagonalisation (Lynch, Rice & Thomas, Numer. Math. 6, 1964).
+//
+// With a constant mass S is a sum of three tensor products of 1D factors:
+// per axis of n cells, D (the difference over a cell's two interior nodes)
+// and A (their sum) give
+//   S0 = (D D^T)(A A^T)(A A^T) + (A A^T)(D D^T)(A A^T) + (A A^T)(A A^T)(D D^T).
+// D D^T + A A^T = W = diag(2, 4, .., 4, 2) (an end cell has one interior
+// node), so D D^T and A A^T share the eigenvectors of the pencil (D D^T, W),
+// which are the DCT-I basis: V_jk = c_k cos(pi j k / (n - 1)) with
+//   V^T W V = I,  V^T D D^T V = diag(s),  V^T A A^T V = diag(1 - s),
+//   s_k = sin^2(pi k / (2 (n - 1))).
+// Hence S0^-1 = V (1 / lambda) V^T in all three axes, with
+//   lambda = sx cy cz + cx sy cz + cx cy sz,  c = 1 - s,
+// and 1 / lambda = 0 on the null space (the constant and the checkerboard
+// modes), which S shares whatever the masses.  For every x,
+// x^T S x / x^T S0 x lies between the smallest and the largest 1 / m, so the
+// iteration count depends on the spread of the node masses only, not on the
+// grid: 4 iterations to 1e-12 where solid and fluid weigh the same, about 15
+// at a density ratio of 2, 57 at 100, where Jacobi-preconditioned CR needs
+// some thousands (the near-checkerboard modes make S's condition number
+// grow as n^4).
+//
+// One application is six dense products along an axis; they run on the
+// matrix cores (FP32 16x16x4) in three kernels: x and y forward, z forward
+// with the scaling and z backward, y and x backward.  The arrays they pass
+// are FP32 with x and y padded to multiples of 16 (pads stay zero).
+#include "esf_fastdiag.h"
+#include "esf_krylov.h"
+
+namespace esf {
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+// packed tables of one axis, padded to P = 16 Q: entry ((m Q + c) 64 + lane) 4
+// + s is V[j][k] with (forward) j = 16 c + 4 (lane / 16) + s, k = 16 m + lane % 16
+// or (backward) j and k exchanged: what lane `lane` feeds to step s of chunk
+// c's four matrix instructions, so a wave reads 1 KB runs.  Then s and 1 - s.
+template <class GridT>
+__device__ __forceinline__ void kFdTables(const GridT& wg, int n, int P, float* fwd, float* bwd,
+                                          float* sv, float* cv) {
+  const int t = wg.block() * blockDim.x + threadIdx.x;
+  const int Q = P >> 4;
+  if (t < P) {
+    const bool in = t < n;
+    const double s = sinpi(0.5 * t / (n - 1)), c = cospi(0.5 * t / (n - 1));
+    sv[t] = in ? (float)(s * s) : 0.0f;
+    // the last mode's cosine is exactly 0 (its modes are null modes)
+    cv[t] = in && t < n - 1 ? (float)(c * c) : 0.0f;
+  }
+  if (t >= P * P) return;
+  const int s = t & 3, lane = (t >> 2) & 63, mc = t >> 8, m = mc / Q, c = mc % Q;
+  const int a = 16 * c + 4 * (lane >> 4) + s, b = 16 * m + (lane & 15);
+  auto value = [&](int j, int k) {
+    if (j >= n || k >= n) return 0.0f;
+    const double norm = sqrt((k == 0 || k == n - 1 ? 0.25 : 0.5) / (n - 1));
+    const long q = (long)j * k % (2 * (n - 1));
+    return (float)(norm * cospi((double)q / (n - 1)));
+  };
+  fwd[t] = value(a, b);
+  bwd[t] = value(b, a);
+}
+ESF_BOUNDS(kFdTables, 256);
+
+__device__ __forceinline__ f4 mfma4(const f4& a, const f4& b, f4 c) {
+#pragma unroll
+  for (int s = 0; s < 4; s++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], c, 0, 0, 0);
+  return c;
+}
+
+__device__ __forceinline__ int waveOf() {
+  return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+
+// The products' blocks: 256 threads, four waves; wave w takes the row tiles
+// (16 rows) w, w + 4, .. of an axis of at most NP = 64 MT nodes, both column
+// tiles of the block's 32 columns per row tile.  An operand lane holds row
+// or column lane % 16 at k = 16 c + 4 (lane / 16) + s of chunk c, s = 0..3;
+// a result lane holds rows 4 (lane / 16) + 0..3 of column lane % 16.
+// LDS rows are NP + 4 floats apart (16-byte reads of 16 rows: no conflict).
+
+// the recursive residual's test: |r|^2 below tol2 |b|^2 ends the solve
+__device__ __forceinline__ bool pcgDone(const PcgTest& t, double rr) {
+  return rr < t.tol2 * t.outer->bnorm * t.outer->bnorm;
+}
+__device__ __forceinline__ void pcgReport(const PcgTest& t, double rr) {
+  t.sc->resnorm = sqrt(rr);
+  t.sc->iter = t.iter;
+  t.sc->done = 1;
+}
+
+// x and y forward: block = (plane z, 32 x modes).  It also tests the
+// recursive residual of the iteration before (the later kernels of a
+// finished solve return at once).
+template <int MT, class GridT>
+__device__ __forceinline__ void kFdXY(const GridT& wg, FdGeom g, const float* __restrict__ r32,
+                                      float* __restrict__ T, const float* __restrict__ fx,
+                                      const float* __restrict__ fy, PcgTest t) {
+  constexpr int LD = 64 * MT + 4;
+  __shared__ __align__(16) float L[32 * LD];
+  __shared__ double red[4];
+  if (t.iter > 0) {
+    if (t.sc->done) return;
+    const double rr = blockTotal(t.nb, t.parts, red);
+    if (pcgDone(t, rr)) {
+      if (wg.block() == 0 && threadIdx.x == 0) pcgReport(t, rr);
+      return;
+    }
+  } else if (wg.block() == 0 && threadIdx.x == 0) {
+    initScalarBlock(t.sc, 0);  // read by the later kernels only
+  }
+  const int lane = threadIdx.x & 63, w = waveOf(), col = lane & 15, gr = lane >> 4;
+  const int z = wg.block() / g.tx, kx0 = 32 * (wg.block() % g.tx);
+  const int QX = g.PX >> 4, QY = g.PY >> 4;
+  const int two = kx0 + 16 < g.PX ? 1 : 0;
+  const long plane = (long)z * g.PY * g.PX;
+  const f4* bx0 = (const f4*)fx + (size_t)(kx0 >> 4) * QX * 64 + lane;
+  const f4* bx1 = bx0 + (size_t)two * QX * 64;
+  f4 acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT; i++) acc[i][0] = acc[i][1] = f4{0, 0, 0, 0};
+  const float* rows = r32 + plane + 4 * gr;
+  for (int c = 0; c < QX; c++) {
+    const f4 b0 = bx0[c * 64], b1 = bx1[c * 64];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int m = w + 4 * i;
+      if (m < QY) {
+        const f4 a = *(const f4*)&rows[(long)(16 * m + col) * g.PX + 16 * c];
+        acc[i][0] = mfma4(a, b0, acc[i][0]);
+        acc[i][1] = mfma4(a, b1, acc[i][1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    const int m = w + 4 * i;
+    if (m < QY) {
+      *(f4*)&L[col * LD + 16 * m + 4 * gr] = acc[i][0];
+      *(f4*)&L[(16 + col) * LD + 16 * m + 4 * gr] = acc[i][1];
+    }
+    acc[i][0] = acc[i][1] = f4{0, 0, 0, 0};
+  }
+  __syncthreads();
+  for (int c = 0; c < QY; c++) {
+    const f4 a0 = *(const f4*)&L[col * LD + 16 * c + 4 * gr];
+    const f4 a1 = *(const f4*)&L[(16 + col) * LD + 16 * c + 4 * gr];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int m = w + 4 * i;
+      if (m < QY) {
+        const f4 b = ((const f4*)fy)[(size_t)(m * QY + c) * 64 + lane];
+        acc[i][0] = mfma4(a0, b, acc[i][0]);
+        acc[i][1] = mfma4(a1, b, acc[i][1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    const int m = w + 4 * i;
+    if (m < QY) {
+      float* o = T + plane + (long)(16 * m + col) * g.PX + kx0 + 4 * gr;
+      *(f4*)o = acc[i][0];
+      if (two) *(f4*)(o + 16) = acc[i][1];
+    }
+  }
+}
+ESF_BOUNDS(kFdXY, 256);
+
+// z forward, 1 / lambda, z backward, in place: block = (y mode, 32 x modes)
+template <int MT, class GridT>
+__device__ __forceinline__ void kFdZ(const GridT& wg, FdGeom g, float* __restrict__ T,
+                                     const float* __restrict__ fz, const float* __restrict__ bz,
+                                     const float* __restrict__ sv, const float* __restrict__ cv,
+                                     const CrScalars* sc) {
+  constexpr int LD = 64 * MT + 4;
+  __shared__ __align__(16) float L[32 * LD];
+  if (sc->done) return;
+  const int lane = threadIdx.x & 63, w = waveOf(), col = lane & 15, gr = lane >> 4;
+  const int ky = wg.block() / g.tx, kx0 = 32 * (wg.block() % g.tx);
+  const int QZ = g.PZ >> 4;
+  const int two = kx0 + 16 < g.PX ? 1 : 0;
+  const long zs = (long)g.PY * g.PX;
+  float* base = T + (long)ky * g.PX + kx0;
+  {
+    const int x4 = 4 * (threadIdx.x & 7);
+    const bool in = x4 < 16 || two;
+    for (int z = threadIdx.x >> 3; z < g.PZ; z += 32) {
+      const f4 v = z < g.nz && in ? *(const f4*)&base[z * zs + x4] : f4{0, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < 4; q++) L[(x4 + q) * LD + z] = v[q];
+    }
+  }
+  f4 acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT; i++) acc[i][0] = acc[i][1] = f4{0, 0, 0, 0};
+  __syncthreads();
+  for (int c = 0; c < QZ; c++) {
+    const f4 b0 = *(const f4*)&L[col * LD + 16 * c + 4 * gr];
+    const f4 b1 = *(const f4*)&L[(16 + col) * LD + 16 * c + 4 * gr];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int m = w + 4 * i;
+      if (m < QZ) {
+        const f4 a = ((const f4*)fz)[(size_t)(m * QZ + c) * 64 + lane];
+        acc[i][0] = mfma4(a, b0, acc[i][0]);
+        acc[i][1] = mfma4(a, b1, acc[i][1]);
+      }
+    }
+  }
+  __syncthreads();
+  {
+    const float sy = sv[g.PX + ky], cy = cv[g.PX + ky];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int kx = kx0 + (two ? 16 * j : 0) + col;
+      const float sx = sv[kx], cx = cv[kx];
+      const float p = sx * cy + cx * sy, q = cx * cy;
+#pragma unroll
+      for (int i = 0; i < MT; i++) {
+        const int m = w + 4 * i;
+        if (m < QZ) {
+          const f4 sz = *(const f4*)&sv[g.PX + g.PY + 16 * m + 4 * gr];
+          const f4 cz = *(const f4*)&cv[g.PX + g.PY + 16 * m + 4 * gr];
+          f4 v = acc[i][j];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float lam = p * cz[e] + q * sz[e];
+            v[e] = lam > 0.0f ? v[e] / lam : 0.0f;
+          }
+          *(f4*)&L[(16 * j + col) * LD + 16 * m + 4 * gr] = v;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; i++) acc[i][0] = acc[i][1] = f4{0, 0, 0, 0};
+  __syncthreads();
+  for (int c = 0; c < QZ; c++) {
+    const f4 a0 = *(const f4*)&L[col * LD + 16 * c + 4 * gr];
+    const f4 a1 = *(const f4*)&L[(16 + col) * LD + 16 * c + 4 * gr];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int m = w + 4 * i;
+      if (m < QZ) {
+        const f4 b = ((const f4*)bz)[(size_t)(m * QZ + c) * 64 + lane];
+        acc[i][0] = mfma4(a0, b, acc[i][0]);
+        acc[i][1] = mfma4(a1, b, acc[i][1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    const int z = 16 * (w + 4 * i) + col;
+    if (z < g.nz) {
+      float* o = base + z * zs + 4 * gr;
+      *(f4*)o = acc[i][0];
+      if (two) *(f4*)(o + 16) = acc[i][1];
+    }
+  }
+}
+ESF_BOUNDS(kFdZ, 256);
+
+// y and x backward: block = (plane z, 32 rows y); z = S0^-1 r in the cells'
+// own layout, and the block's share of r . z
+template <int MT, class GridT>
+__device__ __forceinline__ void kFdYX(const GridT& wg, FdGeom g, const float* __restrict__ T,
+                                      const float* __restrict__ r32, float* __restrict__ zOut,
+                                      const float* __restrict__ by, const float* __restrict__ bx,
+                                      const CrScalars* sc, double* parts) {
+  constexpr int LD = 64 * MT + 4;
+  __shared__ __align__(16) float L[32 * LD];
+  __shared__ double red[4];
+  if (sc->done) return;
+  const int lane = threadIdx.x & 63, w = waveOf(), col = lane & 15, gr = lane >> 4;
+  const int z = wg.block() / g.ty, y0 = 32 * (wg.block() % g.ty);
+  const int QX = g.PX >> 4, QY = g.PY >> 4;
+  const int two = y0 + 16 < g.PY ? 1 : 0;
+  const long plane = (long)z * g.PY * g.PX;
+  const f4* by0 = (const f4*)by + (size_t)(y0 >> 4) * QY * 64 + lane;
+  const f4* by1 = by0 + (size_t)two * QY * 64;
+  f4 acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT; i++) acc[i][0] = acc[i][1] = f4{0, 0, 0, 0};
+  for (int c = 0; c < QY; c++) {
+    const f4 b0 = by0[c * 64], b1 = by1[c * 64];
+    const float* rows = T + plane + (long)(16 * c + 4 * gr) * g.PX + col;
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int m = w + 4 * i;
+      if (m < QX) {
+        f4 a;
+#pragma unroll
+        for (int s = 0; s < 4; s++) a[s] = rows[s * g.PX + 16 * m];
+        acc[i][0] = mfma4(a, b0, acc[i][0]);
+        acc[i][1] = mfma4(a, b1, acc[i][1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    const int m = w + 4 * i;
+    if (m < QX) {
+      *(f4*)&L[col * LD + 16 * m + 4 * gr] = acc[i][0];
+      *(f4*)&L[(16 + col) * LD + 16 * m + 4 * gr] = acc[i][1];
+    }
+    acc[i][0] = acc[i][1] = f4{0, 0, 0, 0};
+  }
+  __syncthreads();
+  for (int c = 0; c < QX; c++) {
+    const f4 b0 = *(const f4*)&L[col * LD + 16 * c + 4 * gr];
+    const f4 b1 = *(const f4*)&L[(16 + col) * LD + 16 * c + 4 * gr];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int m = w + 4 * i;
+      if (m < QX) {
+        const f4 a = ((const f4*)bx)[(size_t)(m * QX + c) * 64 + lane];
+        acc[i][0] = mfma4(a, b0, acc[i][0]);
+        acc[i][1] = mfma4(a, b1, acc[i][1]);
+      }
+    }
+  }
+  double dot = 0;
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    const int x = 16 * (w + 4 * i) + 4 * gr;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int y = y0 + 16 * j + col;
+      if (w + 4 * i < QX && y < g.ny) {
+        const f4 v = acc[i][j];
+        const f4 r = *(const f4*)&r32[plane + (long)y * g.PX + x];
+        float* o = zOut + ((long)z * g.ny + y) * g.nx + x;
+        if ((g.nx & 3) == 0) {
+          if (x < g.nx) *(f4*)o = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            if (x + e < g.nx) o[e] = v[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) dot += (double)v[e] * (double)r[e];
+      }
+    }
+  }
+  double mine[1] = {dot};
+  blockPartialsAt<1>(mine, parts, red, wg.blocks(), wg.block());
+}
+ESF_BOUNDS(kFdYX, 256);
+
+// x += alpha p, r -= alpha q, r in FP32 for the preconditioner, |r|^2;
+// alpha = (r . z) / (p . q).  p . q not above 0 (no direction left, or NaN)
+// ends the solve with done = 2.
+template <class GridT>
+__device__ __forceinline__ void kPcgUpdate(const GridT& wg, FdGeom g, long cells,
+                                           const double* __restrict__ p,
+                                           const double* __restrict__ q, double* __restrict__ x,
+                                           double* __restrict__ r, float* __restrict__ r32,
+                                           int nbQ, const double* __restrict__ partsQ,
+                                           const double* __restrict__ rz, CrScalars* sc,
+                                           double* parts) {
+  __shared__ double red[4];
+  if (sc->done) return;
+  const double pq = blockTotal(nbQ, partsQ, red);
+  const bool ok = pq > 0.0;
+  if (!ok && wg.block() == 0 && threadIdx.x == 0) sc->done = 2;
+  const double alpha = ok ? *rz / pq : 0.0;
+  double rr = 0;
+  const long n2 = (cells + 1) >> 1;
+  for (long t = wg.block() * (long)blockDim.x + threadIdx.x; t < n2;
+       t += (long)wg.blocks() * blockDim.x) {
+    const int c = (int)(2 * t);
+    const int row = c / g.nx, cx = c - row * g.nx, cz = row / g.ny, cy = row - cz * g.ny;
+    float* o = r32 + ((long)cz * g.PY + cy) * g.PX + cx;
+    double2 rv, xv;
+    if (c + 1 < cells) {
+      const double2 pv = *(const double2*)&p[c], qv = *(const double2*)&q[c];
+      rv = *(const double2*)&r[c];
+      xv = *(const double2*)&x[c];
+      xv.x += alpha * pv.x;
+      xv.y += alpha * pv.y;
+      rv.x -= alpha * qv.x;
+      rv.y -= alpha * qv.y;
+      *(double2*)&x[c] = xv;
+      *(double2*)&r[c] = rv;
+      o[0] = (float)rv.x;
+      // the next cell, in this row or at the start of the next
+      float* o1 = o + 1;
+      if (cx + 1 == g.nx)
+        o1 = r32 + (cy + 1 == g.ny ? (long)(cz + 1) * g.PY : (long)cz * g.PY + cy + 1) * g.PX;
+      *o1 = (float)rv.y;
+      rr += rv.x * rv.x;
+      rr += rv.y * rv.y;
+    } else {
+      rv.x = r[c] - alpha * q[c];
+      x[c] += alpha * p[c];
+      r[c] = rv.x;
+      o[0] = (float)rv.x;
+      rr += rv.x * rv.x;
+    }
+  }
+  double mine[1] = {rr};
+  blockPartialsAt<1>(mine, parts, red, wg.blocks(), wg.block());
+}
+ESF_BOUNDS(kPcgUpdate, 256);
+
+// the same test after the last queued iteration, and the scalar block into
+// the host's report slot (one block)
+template <class GridT>
+__device__ __forceinline__ void kPcgTest(const GridT& wg, PcgTest t, CrScalars* hostOut) {
+  __shared__ double red[4];
+  const double rr = blockTotal(t.nb, t.parts, red);
+  if (threadIdx.x != 0) return;
+  if (!t.sc->done && pcgDone(t, rr)) pcgReport(t, rr);
+  *hostOut = *t.sc;
+}
+ESF_BOUNDS(kPcgTest, 256);
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+static int pad16(int n) { return (n + 15) & ~15; }
+
+FdGeom fdGeom(const Dims& d) {
+  FdGeom g;
+  g.nx = d.CX;
+  g.ny = d.CY;
+  g.nz = d.CZ;
+  g.PX = pad16(d.CX);
+  g.PY = pad16(d.CY);
+  g.PZ = pad16(d.CZ);
+  g.tx = cdiv(g.PX, 32);
+  g.ty = cdiv(g.PY, 32);
+  return g;
+}
+
+// the LDS rows hold one axis: at most kFdMax cells per axis
+constexpr int kFdMax = 256;
+
+bool fdFits(const Dims& d) { return std::max(d.CX, std::max(d.CY, d.CZ)) <= kFdMax; }
+
+esf_status fdCreate(esf_ctx* ctx) {
+  const FdGeom g = fdGeom(ctx->d);
+  FastDiag& f = ctx->fd;
+  esf_status st = ESF_OK;
+  const int P[3] = {g.PX, g.PY, g.PZ}, n[3] = {g.nx, g.ny, g.nz};
+  const long padded = (long)g.nz * g.PY * g.PX;
+  if ((st = devAlloc(ctx, &f.r32, padded))) return st;
+  if ((st = devAlloc(ctx, &f.T, padded))) return st;
+  if ((st = devAlloc(ctx, &f.sv, P[0] + P[1] + P[2]))) return st;
+  if ((st = devAlloc(ctx, &f.cv, P[0] + P[1] + P[2]))) return st;
+  f.nbR = std::min(cdiv((ctx->d.cells + 1) / 2, 256), 1024);
+  f.nbZ = g.nz * g.ty;
+  if ((st = devAlloc(ctx, &f.parts, spmvBlocks(ctx) + f.nbR + f.nbZ))) return st;
+  if ((st = devAlloc(ctx, &f.rz, 2))) return st;
+  long off = 0;
+  for (int a = 0; a < 3; a++) {
+    if ((st = devAlloc(ctx, &f.fwd[a], (size_t)P[a] * P[a]))) return st;
+    if ((st = devAlloc(ctx, &f.bwd[a], (size_t)P[a] * P[a]))) return st;
+    launch<ESF_K(kFdTables)>(ctx, dim3(cdiv(P[a] * P[a], 256)), dim3(256), n[a], P[a], f.fwd[a],
+                             f.bwd[a], f.sv + off, f.cv + off);
+    off += P[a];
+  }
+  return hipGetLastError() == hipSuccess ? ESF_OK : ESF_ERR_DEVICE;
+}
+
+template <int MT>
+static void fdApply(esf_ctx* ctx, const FdGeom& g, const PcgTest& t, float* z) {
+  FastDiag& f = ctx->fd;
+  CrScalars* sc = t.sc;
+  launch<ESF_KT(kFdXY, MT)>(ctx, dim3(g.nz * g.tx), dim3(256), g, (const float*)f.r32, f.T,
+                            (const float*)f.fwd[0], (const float*)f.fwd[1], t);
+  launch<ESF_KT(kFdZ, MT)>(ctx, dim3(g.PY * g.tx), dim3(256), g, f.T, (const float*)f.fwd[2],
+                           (const float*)f.bwd[2], (const float*)f.sv, (const float*)f.cv,
+                           (const CrScalars*)sc);
+  launch<ESF_KT(kFdYX, MT)>(ctx, dim3(f.nbZ), dim3(256), g, (const float*)f.T,
+                            (const float*)f.r32, z, (const float*)f.bwd[1],
+                            (const float*)f.bwd[0], (const CrScalars*)sc,
+                            f.parts + spmvBlocks(ctx) + f.nbR);
+}
+
+static PcgTest pcgTest(esf_ctx* ctx, int it, double eps) {
+  // |r| in the recursion differs from |b - S x| by rounding only; a little
+  // below eps, so the true residual checked afterwards passes
+  const double tol = 0.95 * eps;
+  return {ctx->fd.nbR, ctx->fd.parts + spmvBlocks(ctx), tol * tol, it, &ctx->sc[1], &ctx->sc[0]};
+}
+
+void fdTest(esf_ctx* ctx, int it, double eps, CrScalars* hostOut) {
+  launch<ESF_K(kPcgTest)>(ctx, dim3(1), dim3(256), pcgTest(ctx, it, eps), hostOut);
+}
+
+esf_status fdIteration(esf_ctx* ctx, int it, double eps) {
+  const FdGeom g = fdGeom(ctx->d);
+  FastDiag& f = ctx->fd;
+  const int nbQ = spmvBlocks(ctx);
+  double* partsQ = f.parts;
+  double* partsR = partsQ + nbQ;
+  double* partsZ = partsR + f.nbR;
+  CrScalars* sc = &ctx->sc[1];
+  const PcgTest t = pcgTest(ctx, it, eps);
+  float* z = ctx->e32;
+  const int most = std::max(g.PX, std::max(g.PY, g.PZ));
+  if (most <= 64)
+    fdApply<1>(ctx, g, t, z);
+  else if (most <= 128)
+    fdApply<2>(ctx, g, t, z);
+  else
+    fdApply<4>(ctx, g, t, z);
+  // p alternates between two buffers (halo cells read the previous one)
+  double* pOld = it & 1 ? ctx->r2 : ctx->pdir;
+  double* pNew = it & 1 ? ctx->pdir : ctx->r2;
+  const PcgDir dir{it, f.nbZ, partsZ, f.rz};
+  esf_status st = spmvPcg(ctx, pOld, z, pNew, ctx->Ap, sc, dir, partsQ);
+  if (st) return st;
+  launch<ESF_K(kPcgUpdate)>(ctx, dim3(f.nbR), dim3(256), g, ctx->d.cells, (const double*)pNew,
+                            (const double*)ctx->Ap, ctx->lambda, ctx->r, f.r32, nbQ,
+                            (const double*)partsQ, (const double*)(f.rz + (it & 1)), sc, partsR);
+  return hipGetLastError() == hipSuccess ? ESF_OK : ESF_ERR_DEVICE;
+}
+
+}  // namespace esf

@@ -154,6 +154,20 @@ struct DevSolid {
   int *pBin = nullptr, *binItems = nullptr;
 };
 
+// the mixed form's pressure preconditioner (esf_fastdiag.hip): per axis the
+// packed DCT-I tables, forward and backward, the 1D eigenvalues s and 1 - s
+// of all axes one after another, the residual in FP32 and the transforms'
+// array (x and y padded to multiples of 16), the partial sums of p . S p,
+// |r|^2 and r . z, and r . z of the last two iterations
+struct FastDiag {
+  float* fwd[3] = {nullptr, nullptr, nullptr};
+  float* bwd[3] = {nullptr, nullptr, nullptr};
+  float *sv = nullptr, *cv = nullptr, *r32 = nullptr, *T = nullptr;
+  double *parts = nullptr, *rz = nullptr;
+  int nbR = 0, nbZ = 0;
+  int last = 4;  // iterations the last solve took
+};
+
 struct SceneFiber;  // esf_batch.hip: a scene's step inside esf_step_batch
 
 }  // namespace esf
@@ -223,6 +237,7 @@ struct esf_ctx {
   float *D32 = nullptr, *e32 = nullptr, *r32 = nullptr, *r32b = nullptr,
         *p32 = nullptr, *s32 = nullptr, *Ap32 = nullptr, *rhs32 = nullptr;
   float *s32b = nullptr, *Ap32b = nullptr;
+  esf::FastDiag fd;
   bool lambdaInit = false;
   // solid DOF vectors (3*capSolid)
   double *sForce = nullptr, *sMv = nullptr, *sDamped = nullptr,

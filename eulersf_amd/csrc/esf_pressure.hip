@@ -24,6 +24,7 @@
 // ones), as r does.  A true-residual check every 5 iterations, as the
 // reference does.  Block partials are summed by a one-block finisher (fixed
 // order, deterministic).
+#include "esf_fastdiag.h"
 #include "esf_internal.h"
 #include "esf_krylov.h"
 
@@ -36,6 +37,8 @@ enum SpmvMode {
   M_UPDATE = 3,
   M_CHECK = 4,
   M_IR_RESID = 5,
+  M_PCG = 6,        // p = z + beta p, q = S p, p . q (esf_fastdiag.hip)
+  M_PCG_RESID = 7,  // r = b - S x, also in FP32 in the preconditioner's layout
 };
 
 template <typename T>
@@ -61,6 +64,8 @@ struct SpmvArgs {
   int first;         // M_IR_RESID: also compute |b|
   int recursive;     // M_UPDATE: the finisher tests the recursive residual
   CrScalars* hostOut;  // M_CHECK (M_UPDATE when recursive): pinned slot for the scalar block
+  PcgDir dir;        // M_PCG
+  int px, pxy;       // M_PCG_RESID: the padded layout's strides
 };
 
 constexpr int TX = 32, TY = 8;
@@ -112,6 +117,12 @@ __device__ __forceinline__ void kSpmv(const GridT& wg, Dims d, SpmvArgs<T> a, in
   if (MODE == M_UPDATE) {
     alpha = (T)a.sc->alpha;
     beta = (T)a.sc->beta;
+  }
+  if (MODE == M_PCG) {
+    const double rz = blockTotal(a.dir.nb, a.dir.parts, red);
+    const int now = a.dir.iter & 1;
+    if (a.dir.iter > 0) beta = (T)(rz / a.dir.rz[1 - now]);
+    if (wg.block() == 0 && threadIdx.x == 0) a.dir.rz[now] = rz;
   }
   double part0 = 0, part1 = 0, part2 = 0, part3 = 0, part4 = 0;
 
@@ -190,6 +201,8 @@ __device__ __forceinline__ void kSpmv(const GridT& wg, Dims d, SpmvArgs<T> a, in
         P.dd[h] = a.Dinv[c];
       } else if (MODE == M_IR_RESID) {
         P.e[h] = a.e32 ? a.e32[c] : 0.0f;
+      } else if (MODE == M_PCG) {
+        P.e[h] = a.e32[c];
       }
     }
   };
@@ -209,6 +222,10 @@ __device__ __forceinline__ void kSpmv(const GridT& wg, Dims d, SpmvArgs<T> a, in
         } else if (MODE == M_IR_RESID) {
           // x_old (+ e); the owner writes x_new to the other buffer
           if (a.e32) v = v + (T)P.e[h];
+        } else if (MODE == M_PCG) {
+          // p = z + beta p (the first iteration's previous p is not read as
+          // a number: its buffer may hold anything)
+          v = a.dir.iter > 0 ? (T)P.e[h] + beta * P.in[h] : (T)P.e[h];
         }
         L[hIdx[h]] = zok && hVal[h] ? v : (T)0;
       }
@@ -238,7 +255,8 @@ __device__ __forceinline__ void kSpmv(const GridT& wg, Dims d, SpmvArgs<T> a, in
   };
   auto fetchOut = [&](Pre& P, int cz) {
     const long c = (long)min(max(cz, 0), zEnd - 1) * d.cslab + cOff;
-    if (MODE == M_SETUP_R || MODE == M_CHECK || MODE == M_IR_RESID) P.eB = a.b[c];
+    if (MODE == M_SETUP_R || MODE == M_CHECK || MODE == M_IR_RESID || MODE == M_PCG_RESID)
+      P.eB = a.b[c];
     if (MODE == M_SETUP_R || MODE == M_SETUP_S) P.eD = a.D[c];
     if (MODE == M_UPDATE) {
       P.eX = a.x[c];
@@ -398,6 +416,16 @@ __device__ __forceinline__ void kSpmv(const GridT& wg, Dims d, SpmvArgs<T> a, in
             a.r32[c] = (float)rr;
             part0 += (double)rr * (double)rr;
             part1 += (double)P.eB * (double)P.eB;
+          } else if (MODE == M_PCG) {
+            a.p[c] = ownIn;
+            a.out[c] = acc;
+            part0 += (double)ownIn * (double)acc;
+          } else if (MODE == M_PCG_RESID) {
+            const T rr = P.eB - acc;
+            a.r[c] = rr;
+            a.r32[(long)cz * a.pxy + cy * a.px + cx] = (float)rr;
+            part0 += (double)rr * (double)rr;
+            part1 += (double)P.eB * (double)P.eB;
           }
         }
       }
@@ -451,6 +479,9 @@ __device__ __forceinline__ void kSpmv(const GridT& wg, Dims d, SpmvArgs<T> a, in
   if (MODE == M_UPDATE) {
     double mine[5] = {part0, part1, part2, part3, part4};
     blockPartialsAt<5>(mine, a.partials, red, wg.blocks(), wg.block());
+  } else if (MODE == M_PCG) {
+    double mine[1] = {part0};
+    blockPartialsAt<1>(mine, a.partials, red, wg.blocks(), wg.block());
   } else {
     double mine[2] = {part0, part1};
     blockPartialsAt<2>(mine, a.partials, red, wg.blocks(), wg.block());
@@ -595,15 +626,16 @@ esf_status launchSpmv(esf_ctx* ctx, const SpmvArgs<T>& a) {
   tileShape(ctx, sizeof(T) == 8 && MODE == M_UPDATE, tx, ty, tz, layers);
   const int nb = tx * ty * tz;
   const int depth = MODE == M_UPDATE ? ctx->spmvDepthUpdate : ctx->spmvDepthOther;
+  const int cls = MODE > M_IR_RESID ? -1 : MODE + (sizeof(T) == 4 ? 6 : 0);
   if (depth == 3)
-    launchTimed<ESF_KT(kSpmv, T, MODE, 3)>(ctx, MODE + (sizeof(T) == 4 ? 6 : 0), dim3(nb),
-                                           dim3(256), ctx->d, a, tx, ty, tz, layers);
+    launchTimed<ESF_KT(kSpmv, T, MODE, 3)>(ctx, cls, dim3(nb), dim3(256), ctx->d, a, tx, ty, tz,
+                                           layers);
   else if (depth == 2)
-    launchTimed<ESF_KT(kSpmv, T, MODE, 2)>(ctx, MODE + (sizeof(T) == 4 ? 6 : 0), dim3(nb),
-                                           dim3(256), ctx->d, a, tx, ty, tz, layers);
+    launchTimed<ESF_KT(kSpmv, T, MODE, 2)>(ctx, cls, dim3(nb), dim3(256), ctx->d, a, tx, ty, tz,
+                                           layers);
   else
-    launchTimed<ESF_KT(kSpmv, T, MODE, 1)>(ctx, MODE + (sizeof(T) == 4 ? 6 : 0), dim3(nb),
-                                           dim3(256), ctx->d, a, tx, ty, tz, layers);
+    launchTimed<ESF_KT(kSpmv, T, MODE, 1)>(ctx, cls, dim3(nb), dim3(256), ctx->d, a, tx, ty, tz,
+                                           layers);
   // the grid-wide sums of the mode (kSpmv's epilogue partials)
   if constexpr (MODE == M_SETUP_R) launchFinish<F_BNORM, 1>(ctx, nb, a.sc);
   if constexpr (MODE == M_SETUP_S) launchFinish<F_SETUP_S, 2>(ctx, nb, a.sc);
@@ -611,7 +643,7 @@ esf_status launchSpmv(esf_ctx* ctx, const SpmvArgs<T>& a) {
     launchFinish<F_CR, 5>(ctx, nb, a.sc, a.iter, a.recursive, nullptr, a.hostOut);
   if constexpr (MODE == M_CHECK)
     launchFinish<F_CHECK, 1>(ctx, nb, a.sc, a.iter, 0, nullptr, a.hostOut);
-  if constexpr (MODE == M_IR_RESID)
+  if constexpr (MODE == M_IR_RESID || MODE == M_PCG_RESID)
     launchFinish<F_IR, 2>(ctx, nb, a.sc, 0, a.first, nullptr, a.hostOut);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -881,6 +913,85 @@ __device__ __forceinline__ void kZeroF(const GridT& wg, long n, float* a, CrScal
 }
 ESF_BOUNDS(kZeroF, 1024);
 
+esf_status spmvPcg(esf_ctx* ctx, const double* pOld, const float* z, double* pNew, double* q,
+                   CrScalars* sc, const PcgDir& dir, double* parts) {
+  SpmvArgs<double> a{};
+  a.in = pOld;
+  a.e32 = z;
+  a.p = pNew;
+  a.out = q;
+  a.minv = ctx->minv;
+  a.sc = sc;
+  a.dir = dir;
+  a.partials = parts;
+  return launchSpmv<double, M_PCG>(ctx, a);
+}
+
+// the residual b - S lambda for the iterations of fdSolve, and its norm
+// against eps |b| in scalar block 0 (hostOut: that block, pinned)
+static esf_status fdResidual(esf_ctx* ctx, int first, CrScalars* hostOut) {
+  const FdGeom g = fdGeom(ctx->d);
+  SpmvArgs<double> o{};
+  o.minv = ctx->minv;
+  o.b = ctx->b;
+  o.in = ctx->lambda;
+  o.r = ctx->r;
+  o.r32 = ctx->fd.r32;
+  o.px = g.PX;
+  o.pxy = g.PX * g.PY;
+  o.sc = &ctx->sc[0];
+  o.partials = ctx->partials;
+  o.first = first;
+  o.hostOut = hostOut;
+  return launchSpmv<double, M_PCG_RESID>(ctx, o);
+}
+
+// Conjugate gradients preconditioned by fast diagonalisation
+// (esf_fastdiag.hip) from lambda, whose residual fdResidual has formed.
+// *h: scalar block 0 as the last check of the true residual left it; *made
+// iterations in *rounds starts.  It gives up (h->done == 0) past
+// kFdIterations, when the direction breaks down, or when a restart does not
+// halve the residual; lambda then holds the last iterate.
+static esf_status fdSolve(esf_ctx* ctx, double eps, int maxIt, CrScalars* h, int* made,
+                          int* rounds) {
+  // past 200 iterations the node masses spread over more than three
+  // decades, and the Jacobi scaling of the FP32 CR takes them better
+  constexpr int kFdIterations = 200;
+  const int most = std::min(maxIt, kFdIterations);
+  esf_status st;
+  while (!h->done && *made < most) {
+    const double before = h->resnorm;
+    if (*rounds > 0 && (st = fdResidual(ctx, 0, nullptr))) return st;
+    (*rounds)++;
+    // as many iterations as the last solve took are queued before the host
+    // looks, then one or a few at a time; where the residual passes its test
+    // decides the last iteration, however many were queued
+    int it = 0, chunk = std::max(1, ctx->fd.last);
+    while (*made + it < most) {
+      const int upTo = std::min(it + chunk, most - *made);
+      for (; it < upTo; it++)
+        if ((st = fdIteration(ctx, it, eps))) return st;
+      fdTest(ctx, it, eps, &ctx->hostSc[4]);
+      SpmvArgs<double> a{};
+      a.in = ctx->lambda;
+      a.minv = ctx->minv;
+      a.b = ctx->b;
+      a.sc = &ctx->sc[0];
+      a.partials = ctx->partials;
+      a.hostOut = &ctx->hostSc[3];
+      if ((st = launchSpmv<double, M_CHECK>(ctx, a))) return st;
+      if ((st = waitSlot3(ctx, h))) return st;  // also completes report slot 4
+      if (ctx->hostSc[4].done) break;
+      chunk = it < 8 ? 1 : 4;
+    }
+    if (ctx->hostSc[4].done == 1) it = ctx->hostSc[4].iter;
+    *made += it;
+    ctx->fd.last = it;
+    if (!(h->resnorm < 0.5 * before)) break;
+  }
+  return ESF_OK;
+}
+
 // Mixed-precision pressure solve: FP32 CR on S (FP32 minv, FP32 vectors,
 // FP64 inner products) inside FP64 iterative refinement.  The outer
 // residual b - S x, the correction x += e and |r| stay in FP64.
@@ -901,10 +1012,20 @@ esf_status mixedSolve(esf_ctx* ctx, double eps, int maxIt, int* iters, bool* con
   o.partials = ctx->partials;
   o.first = 1;
   o.hostOut = &ctx->hostSc[3];
-  if ((st = launchSpmv<double, M_IR_RESID>(ctx, o))) return st;
   CrScalars h;
-  if ((st = waitSlot3(ctx, &h))) return st;
   int outer = 0, inner = 0;
+  bool residual = true;  // form the residual the refinement starts from
+  if (ctx->fd.T) {
+    if ((st = fdResidual(ctx, 1, &ctx->hostSc[3]))) return st;
+    if ((st = waitSlot3(ctx, &h))) return st;
+    if (!h.done && (st = fdSolve(ctx, eps, maxIt, &h, &inner, &outer))) return st;
+    residual = !h.done && inner < maxIt;
+  }
+  if (residual) {
+    if ((st = launchSpmv<double, M_IR_RESID>(ctx, o))) return st;
+    if ((st = waitSlot3(ctx, &h))) return st;
+  }
+  bool operands = false;
   // refinement rounds: each gains roughly the FP32 solve's attainable
   // reduction (about eps32 * cond on the smooth modes), so an ill-conditioned
   // cold start needs many; the total FP32 iterations stay capped by maxIt
@@ -921,7 +1042,8 @@ esf_status mixedSolve(esf_ctx* ctx, double eps, int maxIt, int* iters, bool* con
     // earlier, slower builds measured 0.3 / 0.1 / 0.03 well below 0.5.
     double need = h.resnorm > 0 ? 0.7 * eps * h.bnorm / h.resnorm : 1.0;
     double innerEps = std::min(0.5, std::max(need, ctx->p.inner_eps));
-    if (outer == 0) {
+    if (!operands) {
+      operands = true;
       // the inner solve's operands: minv in FP32, and the diagonal where
       // the step left it for here
       if (ctx->diagPending) {

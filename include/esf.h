@@ -54,7 +54,10 @@ typedef int esf_status;
 
 /* precision of the pressure solve */
 #define ESF_PLAIN_FP64 0  /* CR in FP64, the reference's algorithm */
-#define ESF_MIXED 1       /* FP32 CR inside FP64 iterative refinement */
+#define ESF_MIXED 1       /* FP64 CG preconditioned in FP32 (fast
+                             diagonalisation); grids past 256 cells per axis,
+                             and masses spread too far for it, FP32 CR inside
+                             FP64 iterative refinement */
 
 typedef struct {
   int xres, yres, zres; /* node counts ("xRes","yRes","zRes") */
@@ -97,8 +100,8 @@ typedef struct {
   int iterations[3];      /* solid solve 1, pressure solve, solid solve 2 */
   int converged[3];
   double rel_residual[3]; /* true |Ax-b|/|b| at exit, FP64 */
-  int refinements;        /* mixed: outer FP64 refinement steps */
-  int inner_iterations;   /* mixed: FP32 iterations summed over refinements */
+  int refinements;        /* mixed: starts of the solve from a true residual */
+  int inner_iterations;   /* mixed: iterations summed over those */
   double dt;              /* the substep's dt */
   int n_solid_nodes;      /* solid DOF nodes this step */
   int n_solid_cells;      /* valid solid cells (all solids) this step */
@@ -351,9 +354,9 @@ esf_status esf_pressure_solve(esf_ctx* ctx, const double* b, double* x,
 /* Measurement entry point, no reference counterpart (the isolated-system
  * benchmark): solvePCR on S x = b with b (ESF_F_PRESSURE_RHS) and the start
  * x (ESF_F_LAMBDA) already resident, D from the last esf_pressure_diag /
- * esf_forces, in the context's precision (ESF_MIXED: FP32 CR inside FP64
- * refinement).  iterations: CR iterations (mixed: FP32 ones summed);
- * refinements: outer FP64 rounds (0 in FP64); device_ms: the solve's device
+ * esf_forces, in the context's precision.  iterations: CR iterations
+ * (mixed: summed over its starts); refinements: starts from a true residual
+ * (0 in FP64); device_ms: the solve's device
  * time between HIP events on the context stream.  The solution stays in
  * ESF_F_LAMBDA. */
 esf_status esf_pressure_solve_resident(esf_ctx* ctx, double eps, int max_it,

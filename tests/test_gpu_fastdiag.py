@@ -1,0 +1,99 @@
+"""The mixed form's pressure solve on grids at the edges of its tiles: the
+fast-diagonalisation preconditioner is the exact inverse where every interior
+node has one mass, so its error per iteration is FP32 rounding alone; where
+masses differ the solve still ends at the true residual."""
+import numpy as np
+import pytest
+
+from eulersf_amd.cfg import scene_cfg
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def esf():
+    import eulersf_amd
+    eulersf_amd.load()
+    return eulersf_amd
+
+
+def box_cfg(cells, spheres, **kw):
+    n = max(cells)
+    text = scene_cfg(n, spheres, **kw)
+    for axis, c in zip("xyz", cells):
+        text = text.replace("%sRes = %d" % (axis, n + 1), "%sRes = %d" % (axis, c + 1))
+    return text
+
+
+def schur(x, minv):
+    """J M^-1 J^T x in 64 bits: minv per node (z, y, x), 0 on the boundary"""
+    nz, ny, nx = x.shape
+    corners = [(oz, oy, ox) for oz in (0, 1) for oy in (0, 1) for ox in (0, 1)]
+    w = np.zeros((3,) + minv.shape)
+    at = {o: tuple(slice(a, a + n) for a, n in zip(o, x.shape)) for o in corners}
+    for o in corners:
+        for c in range(3):
+            w[(c,) + at[o]] += x if o[2 - c] else -x
+    w *= minv
+    y = np.zeros_like(x)
+    for o in corners:
+        for c in range(3):
+            y += w[(c,) + at[o]] if o[2 - c] else -w[(c,) + at[o]]
+    return y
+
+
+def solve(esf, cells, spheres, eps, seed, max_it=1000):
+    A = esf._abi
+    g = esf.CoupledIntegrator3D.from_cfg_text(box_cfg(cells, spheres, eps=eps), esf.ESF_MIXED)
+    g.forces()
+    g.pressureDiag()
+    nx, ny, nz = cells
+    minv = g.download(A.F_MINV).reshape(nz + 1, ny + 1, nx + 1).copy()
+    for a in range(3):
+        edge = [slice(None)] * 3
+        for e in (0, -1):
+            edge[a] = e
+            minv[tuple(edge)] = 0
+    b = schur(np.random.default_rng(seed).standard_normal((nz, ny, nx)), minv)
+    g.upload(A.F_PRESSURE_RHS, b.reshape(-1))
+    g.upload(A.F_LAMBDA, np.zeros(b.size))
+    it, ref, rr, ms, st = g.pressureSolveResident(eps, max_it)
+    x = g.download(A.F_LAMBDA).reshape(b.shape)
+    g.close()
+    true = np.linalg.norm(b - schur(x, minv)) / np.linalg.norm(b)
+    return it, st, true
+
+
+# one and two 16-wide tiles of a 32-wide block, one cell past each, the edges
+# of the three LDS row lengths (64, 128, 256 cells), odd and flat boxes
+@pytest.mark.parametrize("cells", [(3, 3, 3), (16, 16, 16), (17, 15, 33), (32, 48, 31), (64, 5, 64),
+                                   (65, 63, 9), (128, 16, 7), (9, 129, 128), (7, 20, 256),
+                                   (256, 3, 18)])
+def test_one_mass_solves_in_the_roundings_of_fp32(esf, cells):
+    """With one mass the preconditioned operator is the identity up to FP32
+    rounding: six products over n <= 256 terms, each off by at most about
+    n 2^-24 = 1.5e-5 of its operands' norms, so the residual falls by at
+    least 1e-4 per iteration and three iterations pass 1e-10."""
+    it, st, true = solve(esf, cells, [], 1e-10, 3)
+    print(cells, it, true, flush=True)
+    assert st == 0 and it <= 3
+    assert true < 1e-10
+
+
+@pytest.mark.parametrize("density", [50.0, 400.0, 3000.0])
+def test_masses_that_differ(esf, density):
+    """conjugate gradients at condition number k = the ratio of the masses
+    need at most sqrt(k) ln(2 / eps) / 2 iterations, up to rounding"""
+    ball = {"center": (0.5, 0.6, 0.5), "radius": 0.17, "density": density}
+    it, st, true = solve(esf, (40, 37, 45), [ball], 1e-10, 5)
+    k = max(density / 1000.0, 1000.0 / density)
+    print(density, it, true, flush=True)
+    assert st == 0 and true < 1e-10
+    assert it <= 1.1 * np.sqrt(1.05 * k) * np.log(2e10 * k) / 2 + 3
+
+
+def test_a_grid_past_the_tables_takes_the_refinement(esf):
+    # (Jacobi-preconditioned: some thousands of iterations)
+    it, st, true = solve(esf, (260, 6, 5), [], 1e-8, 4, max_it=100000)
+    print(it, true, flush=True)
+    assert st == 0 and true < 1e-8
