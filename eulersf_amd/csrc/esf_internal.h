@@ -223,6 +223,8 @@ struct esf_ctx {
   int* swFirst = nullptr;
   double2* swCoef = nullptr;
   size_t swCoefCap = 0;
+  unsigned long long* swEdge = nullptr;  // values handed between a sweep's waves
+  long swEdgeCap = 0;
   int *binCount = nullptr, *binStart = nullptr, *binCursor = nullptr, *binBlocks = nullptr;
   double* randTable = nullptr;
   long randCap = 0;

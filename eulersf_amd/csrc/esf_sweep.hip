@@ -12,15 +12,17 @@
 // neighbours visited before it along i, j and k (or, for the faces, only
 // what the previous loop nest wrote).  A node's new value therefore depends
 // only on those three, so the nodes of one plane i' + j' + k' = p (primed:
-// positions along the sweep's directions) are independent and the planes
-// run in order: one workgroup walks the planes with a barrier between
-// them, and every node gets the reference's value by the reference's
-// arithmetic.  sweepOnePass also carries three flags across the whole pass
+// positions along the sweep's directions) are independent, and every node
+// gets the reference's value by the reference's arithmetic whatever order
+// respects the three.  kPencil lets one wave march along i' with 8 x 8 rows
+// (j', k'), the waves passing their edge rows on through memory.
+// sweepOnePass also carries three flags across the whole pass
 // (solvableX/Y/Z: once cleared they stay cleared).  Whether a node clears
 // one depends on phi and the mass only, never on the field being swept, so
 // a parallel prepass finds, per flag, the first node in loop order that
 // clears it (an integer atomic minimum); a node's flag is then "its loop
-// position comes before that one".
+// position comes before that one".  The four rounds of a pass share its
+// flags and coefficients, formed once.
 //
 // These are host-side stages of the reference's finalize that the step does
 // not run; the entry points serve a host integrator that keeps them.
@@ -32,8 +34,6 @@
 namespace esf {
 
 namespace {
-
-constexpr int kWaveThreads = 1024;
 
 struct SweepBox {
   int X, Y, Z;
@@ -72,32 +72,295 @@ __device__ __forceinline__ void kSdfInit(const GridT& wg, long n, int X, int Y,
 }
 ESF_BOUNDS(kSdfInit, 1024);
 
-// sweepPhi's sweep s, one workgroup, plane by plane
-template <class GridT>
-__device__ __forceinline__ void kPhiWave(const GridT& wg, SweepBox b, Sweep s,
-                                         const double* __restrict__ mass, double* phi) {
-  const int planes = s.ni + s.nj + s.nk - 2;
-  for (int p = 0; p < planes; p++) {
-    // the (j', k') rectangle that can hold a node of plane p
-    const int jLo = max(0, p - (s.ni - 1) - (s.nk - 1)), jHi = min(s.nj - 1, p);
-    const int kLo = max(0, p - (s.ni - 1) - (s.nj - 1)), kHi = min(s.nk - 1, p);
-    const int wj = jHi - jLo + 1, wk = kHi - kLo + 1;
-    const int jk = wj > 0 && wk > 0 ? wj * wk : 0;
-    for (int t = threadIdx.x; t < jk; t += blockDim.x) {
-      const int jp = jLo + t % wj, kp = kLo + t / wj, ip = p - jp - kp;
-      if (ip < 0 || ip >= s.ni) continue;
-      const int i = s.i0 + s.di * ip, j = s.j0 + s.dj * jp, k = s.k0 + s.dk * kp;
-      const long c = nodeAt(b, i, j, k);
-      // the mass and the four phi values in one round of loads
-      const double mc = mass[c], pa = phi[nodeAt(b, i - s.di, j, k)],
-                   pb = phi[nodeAt(b, i, j - s.dj, k)], pe = phi[nodeAt(b, i, j, k - s.dk)],
-                   pc = phi[c];
-      if (mc == 0) phi[c] = solveDistance(pa, pb, pe, pc);
+// solveDistance with its three candidates formed side by side (the sweep's
+// time is this chain's latency) and chosen as the reference's loop does; a
+// division by 3 is the rounded reciprocal's product corrected by one fused
+// step (Markstein: correctly rounded for finite quotients), one by 2 or 1
+// exact
+__device__ __forceinline__ double solveDistance3(double p, double q, double r, double v) {
+  const double d0 = fmin(p, fmin(q, r)), d2 = fmax(p, fmax(q, r));
+  const double d1 = p + q + r - d0 - d2;
+  const double c0 = d0 * d0 - 1.0, b1 = d1 + d0, c1 = d1 * d1 + c0;
+  const double b2 = d2 + b1, c2 = d2 * d2 + c1;
+  const double disc2 = b2 * b2 - 3.0 * c2, disc1 = b1 * b1 - 2.0 * c1, disc0 = d0 * d0 - c0;
+  constexpr double third = 1.0 / 3.0;
+  const double n2 = b2 + sqrt(disc2), q2 = n2 * third;
+  double nd = fma(fma(-3.0, q2, n2), third, q2);
+  const double nd1 = (b1 + sqrt(disc1)) * 0.5, nd0 = d0 + sqrt(disc0);
+  if (disc2 < 0.0 || nd < d2) {
+    if (disc1 > 0.0) nd = nd1;
+    if (disc1 < 0.0 || nd < d1) {
+      if (disc0 > 0.0) nd = nd0;
     }
-    __syncthreads();
+  }
+  return nd < v ? nd : v;
+}
+
+// One ordered sweep (phi: sweepPhi, else sweepOnePass) by blocks of 8 x 8
+// rows: lane (j, k) of the block's first wave has row j' = 8 J + j,
+// k' = 8 K + k of tile (J, K) and updates i' = step - j - k, so the rows
+// before it along j' and k' are one step ahead and their values come from
+// lanes l - 1 and l - 8.  Row j = 7 (k = 7) hands its values to tile (J + 1,
+// K) ((J, K + 1)) in `edge`: each double as two words of 32 bits with a tag
+// that only this sweep uses, stored and loaded at device scope, so a reader
+// knows a word's value as soon as it sees it and no fence is needed.  A block
+// takes its tile by a ticket, in an order in which tiles depend only on
+// earlier ones: a tile that waits waits for tiles that are running.
+//
+// What bounds a sweep is the chain of its planes (i' + j' + k') and the
+// tiles' hand-overs, so the updating wave must not wait for memory: the
+// second wave reads the rows' old values and operands ahead, the third asks
+// for the edge words, both through rings in LDS, and the first only stores.
+// (One wave doing all three waits for its stores whenever it looks for an
+// edge word: 319 us per sweep of phi over the box of two balls at 96^3
+// cells, 173 us this way.  One workgroup walking the planes of the whole box
+// with a barrier each took 2 us per plane, 540 us at 64^3 cells, where this
+// takes 111 us.)
+constexpr int kRows = 8;
+constexpr int kRing = 16;
+// tickets of the sweeps of one call, and the tags' epoch before them
+constexpr int kSweepTickets = 32;
+
+struct SweepSync {
+  int* ints;           // epoch, then a ticket per sweep
+  unsigned long long* edge;
+  int slot;            // this sweep's ticket
+};
+
+template <class GridT>
+__device__ __forceinline__ void kSweepStart(const GridT& wg, int* ints) {
+  const int t = threadIdx.x;
+  if (t < kSweepTickets) ints[1 + t] = 0;
+  // (a fresh buffer is 0: the epoch steps over tag 0)
+  if (t == kSweepTickets) {
+    const unsigned e = (unsigned)ints[0] + kSweepTickets;
+    ints[0] = (int)(e < (unsigned)kSweepTickets ? (unsigned)kSweepTickets : e);
   }
 }
-ESF_BOUNDS(kPhiWave, kWaveThreads);
+ESF_BOUNDS(kSweepStart, 64);
+
+// a counter in LDS, and everything this wave wrote to LDS before it
+__device__ __forceinline__ int ldsCount(const int* c) {
+  const int v = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  asm volatile("" ::: "memory");
+  return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ void ldsPublish(int* c, int v) {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __hip_atomic_store(c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <int C, bool PHI, class GridT>
+__device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
+                                        const double* __restrict__ mass,
+                                        const double2* __restrict__ coef, double* f,
+                                        SweepSync sync) {
+  constexpr int E = PHI ? 2 : 5;  // values per node read ahead: field, mass / alpha, beta
+  __shared__ double ring[kRing * E * 64];
+  __shared__ double ering[kRing * 16 * C];
+  __shared__ int cnt[4];  // steps of the ring filled, of the edges, done; the tile
+  const int lane = threadIdx.x & 63;
+  const int role = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
+  if (threadIdx.x == 0) cnt[3] = atomicAdd(&sync.ints[1 + sync.slot], 1);
+  __syncthreads();
+  const int tile = __builtin_amdgcn_readfirstlane(cnt[3]);
+  const int nJ = (s.nj + kRows - 1) / kRows, nK = (s.nk + kRows - 1) / kRows;
+  if (tile >= nJ * nK) return;
+  const unsigned long long tag = (unsigned long long)(unsigned)(sync.ints[0] + sync.slot) << 32;
+  const int J = tile % nJ, K = tile / nJ;
+  const long strideJ = (long)s.dj * b.X, strideK = (long)s.dk * b.X * b.Y;
+  // edge words: ni x 8 rows x C doubles of 2 words per tile with a next one
+  // along j', then the same along k'
+  const long perTile = (long)s.ni * kRows * 2 * C;
+  const int fromJ = K * (nJ - 1) + J - 1, fromK = (nJ - 1) * nK + (K - 1) * nJ + J;
+  const int steps = s.ni + 2 * (kRows - 1);
+
+  if (role == 2) {
+    // edge streams: 0..7 row j' - 1 of lanes (0, k), 8..15 row k' - 1 of lanes
+    // (j, 0), from the tile before or, at the box's edge, from the field,
+    // where no node of this sweep lies; lane 16 u + stream looks at steps
+    // u and u + 4 beyond those handed on
+    const int str = lane & 15, u = lane >> 4;
+    const bool forJ = str < kRows;
+    const int q8 = str & 7, ej = forJ ? 0 : q8, ek = forJ ? q8 : 0;
+    const bool mem = forJ ? J == 0 : K == 0;
+    const bool row = kRows * J + ej < s.nj && kRows * K + ek < s.nk;
+    const int eJ = min(kRows * J + ej, s.nj - 1), eK = min(kRows * K + ek, s.nk - 1);
+    const long mAt = nodeAt(b, s.i0, s.j0 + s.dj * eJ, s.k0 + s.dk * eK) -
+                     (forJ ? strideJ : strideK);
+    const unsigned long long* const in =
+        sync.edge + (forJ ? perTile * fromJ : perTile * fromK) + 2 * C * q8;
+    int p = 0;
+    while (p < steps) {
+      const int room = ldsCount(&cnt[2]) + kRing - p;
+      if (room <= 0) {
+        __builtin_amdgcn_s_sleep(1);
+        continue;
+      }
+      unsigned long long w[2][2 * C];
+      bool ready[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int i = p + u + 4 * h - q8;
+        const bool need = row && i >= 0 && i < s.ni;
+#pragma unroll
+        for (int q = 0; q < 2 * C; q++) w[h][q] = tag;
+        if (need && mem) {
+          const long c = mAt + (long)s.di * i;
+#pragma unroll
+          for (int q = 0; q < C; q++) {
+            const double v = f[C * c + q];
+            w[h][2 * q] = tag | (unsigned)__double2loint(v);
+            w[h][2 * q + 1] = tag | (unsigned)__double2hiint(v);
+          }
+        } else if (need) {
+          const unsigned long long* e = in + (long)i * kRows * 2 * C;
+#pragma unroll
+          for (int q = 0; q < 2 * C; q++)
+            w[h][q] = __hip_atomic_load(e + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        ready[h] = true;
+#pragma unroll
+        for (int q = 0; q < 2 * C; q++) ready[h] = ready[h] && (w[h][q] >> 32) == (tag >> 32);
+      }
+      // the leading steps whose 16 streams are all there, as far as the ring
+      // has room
+      const unsigned long long m0 = __ballot(ready[0]), m1 = __ballot(ready[1]);
+      int n = 0;
+      for (int t = 0; t < 8; t++) {
+        const unsigned long long m = t < 4 ? m0 >> (16 * t) : m1 >> (16 * (t - 4));
+        if ((m & 0xffff) != 0xffff) break;
+        n = t + 1;
+      }
+      n = min(n, room);
+      if (n == 0) continue;
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        if (u + 4 * h < n) {
+          double* o = ering + (((p + u + 4 * h) & (kRing - 1)) * 16 + str) * C;
+#pragma unroll
+          for (int q = 0; q < C; q++)
+            o[q] = __hiloint2double((int)(unsigned)w[h][2 * q + 1], (int)(unsigned)w[h][2 * q]);
+        }
+      p += n;
+      ldsPublish(&cnt[1], p);
+    }
+    return;
+  }
+
+  const int j = lane & 7, k = lane >> 3;
+  const int jp = kRows * J + j, kp = kRows * K + k;
+  const bool row = jp < s.nj && kp < s.nk;
+  const int jc = min(jp, s.nj - 1), kc = min(kp, s.nk - 1);
+  const long at = nodeAt(b, s.i0, s.j0 + s.dj * jc, s.k0 + s.dk * kc);
+
+  if (role == 1) {
+    const long cAt = ((long)kc * s.nj + jc) * s.ni;  // coef: loop position of the row
+    constexpr int G = 4;
+    double v[G][E];
+    auto fetch = [&](int step) {
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int ic = min(max(step + u - j - k, 0), s.ni - 1);
+        const long c = at + (long)s.di * ic;
+#pragma unroll
+        for (int q = 0; q < C; q++) v[u][q] = f[C * c + q];
+        if (PHI) {
+          v[u][1] = mass[c];
+        } else {
+          const double2 ab = coef[cAt + ic];
+          v[u][E - 2] = ab.x;
+          v[u][E - 1] = ab.y;
+        }
+      }
+    };
+    for (int step = 0; step < steps; step += G) {
+      // the old values must be read before the first wave overwrites them:
+      // it does so only after this group is handed on
+      fetch(step);
+      while (ldsCount(&cnt[2]) + kRing < step + G) __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+      for (int u = 0; u < G; u++)
+#pragma unroll
+        for (int e = 0; e < E; e++)
+          ring[(((step + u) & (kRing - 1)) * E + e) * 64 + lane] = v[u][e];
+      ldsPublish(&cnt[0], step + G);
+    }
+    return;
+  }
+
+  unsigned long long* const outJ = sync.edge + perTile * (fromJ + 1) + 2 * C * k;
+  unsigned long long* const outK = sync.edge + perTile * (fromK + nJ) + 2 * C * j;
+  const bool giveJ = j == kRows - 1 && J + 1 < nJ && row;
+  const bool giveK = k == kRows - 1 && K + 1 < nK && row;
+  double last[C], cur[C];  // the values at i' - 1 and of the last step
+#pragma unroll
+  for (int q = 0; q < C; q++) {
+    last[q] = f[C * (at - s.di) + q];
+    cur[q] = 0;
+  }
+  int have = 0;
+  for (int step = 0; step < steps; step++) {
+    while (have <= step) have = min(ldsCount(&cnt[0]), ldsCount(&cnt[1]));
+    const double* o = ring + (step & (kRing - 1)) * E * 64 + lane;
+    const double* e = ering + (step & (kRing - 1)) * 16 * C;
+    double own[E], nj[C], nk[C];
+#pragma unroll
+    for (int q = 0; q < E; q++) own[q] = o[64 * q];
+#pragma unroll
+    for (int q = 0; q < C; q++) {
+      const double ej = e[k * C + q], ek = e[(kRows + j) * C + q];
+      const double sj = dppMov<0x111>(cur[q]), sk = __shfl_up(cur[q], kRows, 64);  // row_shr:1
+      nj[q] = j == 0 ? ej : sj;
+      nk[q] = k == 0 ? ek : sk;
+    }
+    const int i = step - j - k;
+    const bool act = row && i >= 0 && i < s.ni;
+    double nv[C];
+    if (PHI) {
+      nv[0] = own[1] == 0 ? solveDistance3(last[0], nj[0], nk[0], own[0]) : own[0];
+    } else {
+      const double alpha = own[E - 2], beta = own[E - 1], gamma = 1 - alpha - beta;
+      const bool upd = !isnan(alpha);  // else not updated in this pass
+#pragma unroll
+      for (int q = 0; q < C; q++) {
+        const double v = alpha * last[q] + beta * nj[q] + gamma * nk[q];
+        nv[q] = upd ? v : own[q];
+      }
+    }
+    if (act) {
+      const long c = at + (long)s.di * i;
+#pragma unroll
+      for (int q = 0; q < C; q++) {
+        f[C * c + q] = nv[q];
+        last[q] = nv[q];
+        cur[q] = nv[q];
+      }
+      if (giveJ || giveK) {
+#pragma unroll
+        for (int q = 0; q < C; q++) {
+          const unsigned long long lo = tag | (unsigned)__double2loint(nv[q]);
+          const unsigned long long hi = tag | (unsigned)__double2hiint(nv[q]);
+          const long w = (long)i * kRows * 2 * C + 2 * q;
+          if (giveJ) {
+            __hip_atomic_store(outJ + w, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(outJ + w + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          if (giveK) {
+            __hip_atomic_store(outK + w, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(outK + w + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+      }
+    }
+    ldsPublish(&cnt[2], step + 1);
+  }
+}
+ESF_BOUNDS(kPencil, 192);
 
 // sweepOnePass's per-node decisions, from phi and the mass only:
 // returns false where the node is not updated; clear* say whether the node
@@ -133,38 +396,55 @@ __device__ inline bool passNode(const SweepBox& b, const Sweep& s, const double*
   return true;
 }
 
-// the first node, in loop order, that clears each flag
+// sweepVectorField's eight passes, all of the same lengths
+struct Passes {
+  Sweep s[8];
+};
+
+// per pass the first node, in loop order, that clears each flag; blocks
+// [p per, (p + 1) per) take pass p
 template <class GridT>
-__device__ __forceinline__ void kPassFlags(const GridT& wg, SweepBox b, Sweep s,
+__device__ __forceinline__ void kPassFlags(const GridT& wg, SweepBox b, Passes ps, int per,
                                            const double* __restrict__ mass,
                                            const double* __restrict__ phi, int* first) {
-  const long n = (long)s.ni * s.nj * s.nk;
-  for (long t = wg.block() * (long)blockDim.x + threadIdx.x; t < n;
-       t += (long)wg.blocks() * blockDim.x) {
-    const int ip = (int)(t % s.ni), jp = (int)((t / s.ni) % s.nj), kp = (int)(t / ((long)s.ni * s.nj));
+  const int p = wg.block() / per;
+  const Sweep s = ps.s[p];
+  const int n = s.ni * s.nj * s.nk;
+  int m[3] = {INT_MAX, INT_MAX, INT_MAX};
+  for (int t = (wg.block() % per) * blockDim.x + threadIdx.x; t < n; t += per * blockDim.x) {
+    const int q = t / s.ni, ip = t - q * s.ni, kp = q / s.nj, jp = q - kp * s.nj;
     PassNode o;
     passNode(b, s, mass, phi, s.i0 + s.di * ip, s.j0 + s.dj * jp, s.k0 + s.dk * kp, o);
-    if (o.clearX) atomicMin(&first[0], (int)t);
-    if (o.clearY) atomicMin(&first[1], (int)t);
-    if (o.clearZ) atomicMin(&first[2], (int)t);
+    if (o.clearX) m[0] = min(m[0], t);
+    if (o.clearY) m[1] = min(m[1], t);
+    if (o.clearZ) m[2] = min(m[2], t);
+  }
+  // one atomic per wave and flag: with one per node the three words' atomics
+  // alone took 24 us per pass over a 92^3 box
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    for (int off = 32; off; off >>= 1) m[a] = min(m[a], __shfl_xor(m[a], off, 64));
+    if ((threadIdx.x & 63) == 0 && m[a] != INT_MAX) atomicMin(&first[3 * p + a], m[a]);
   }
 }
 ESF_BOUNDS(kPassFlags, 1024);
 
-// every node's coefficients for the pass, from the flags' first clearing
+// every node's coefficients for each pass, from the flags' first clearing
 // nodes: alpha and beta where the node is updated, NaN in alpha where it
-// is not (indexed by loop position), so the wave below reads them together
-// with the neighbours' field values in one round of loads
+// is not (indexed by loop position), so the pass reads them together with
+// the neighbours' field values in one round of loads
 template <class GridT>
-__device__ __forceinline__ void kPassCoef(const GridT& wg, SweepBox b, Sweep s,
+__device__ __forceinline__ void kPassCoef(const GridT& wg, SweepBox b, Passes ps, int per,
                                           const double* __restrict__ mass,
                                           const double* __restrict__ phi,
                                           const int* __restrict__ first, double2* coef) {
-  const long n = (long)s.ni * s.nj * s.nk;
-  const int fx = first[0], fy = first[1], fz = first[2];
-  for (long t = wg.block() * (long)blockDim.x + threadIdx.x; t < n;
-       t += (long)wg.blocks() * blockDim.x) {
-    const int ip = (int)(t % s.ni), jp = (int)((t / s.ni) % s.nj), kp = (int)(t / ((long)s.ni * s.nj));
+  const int p = wg.block() / per;
+  const Sweep s = ps.s[p];
+  const int n = s.ni * s.nj * s.nk;
+  coef += (long)p * n;
+  const int fx = first[3 * p], fy = first[3 * p + 1], fz = first[3 * p + 2];
+  for (int t = (wg.block() % per) * blockDim.x + threadIdx.x; t < n; t += per * blockDim.x) {
+    const int q = t / s.ni, ip = t - q * s.ni, kp = q / s.nj, jp = q - kp * s.nj;
     PassNode o;
     double2 ab = make_double2(NAN, 0.0);
     if (passNode(b, s, mass, phi, s.i0 + s.di * ip, s.j0 + s.dj * jp, s.k0 + s.dk * kp, o)) {
@@ -182,40 +462,6 @@ __device__ __forceinline__ void kPassCoef(const GridT& wg, SweepBox b, Sweep s,
   }
 }
 ESF_BOUNDS(kPassCoef, 1024);
-
-// the pass itself, one workgroup, plane by plane
-template <class GridT>
-__device__ __forceinline__ void kPassWave(const GridT& wg, SweepBox b, Sweep s,
-                                          const double2* __restrict__ coef, double* field) {
-  const int planes = s.ni + s.nj + s.nk - 2;
-  for (int p = 0; p < planes; p++) {
-    const int jLo = max(0, p - (s.ni - 1) - (s.nk - 1)), jHi = min(s.nj - 1, p);
-    const int kLo = max(0, p - (s.ni - 1) - (s.nj - 1)), kHi = min(s.nk - 1, p);
-    const int wj = jHi - jLo + 1, wk = kHi - kLo + 1;
-    const int jk = wj > 0 && wk > 0 ? wj * wk : 0;
-    for (int t = threadIdx.x; t < jk; t += blockDim.x) {
-      const int jp = jLo + t % wj, kp = kLo + t / wj, ip = p - jp - kp;
-      if (ip < 0 || ip >= s.ni) continue;
-      const int i = s.i0 + s.di * ip, j = s.j0 + s.dj * jp, k = s.k0 + s.dk * kp;
-      const double2 ab = coef[(kp * s.nj + jp) * (long)s.ni + ip];
-      const long c = 3 * nodeAt(b, i, j, k), a = 3 * nodeAt(b, i - s.di, j, k),
-                 bb = 3 * nodeAt(b, i, j - s.dj, k), e = 3 * nodeAt(b, i, j, k - s.dk);
-      double fa[3], fb[3], fe[3];
-#pragma unroll
-      for (int q = 0; q < 3; q++) {
-        fa[q] = field[a + q];
-        fb[q] = field[bb + q];
-        fe[q] = field[e + q];
-      }
-      if (isnan(ab.x)) continue;  // not updated in this pass
-      const double alpha = ab.x, beta = ab.y, gamma = 1 - alpha - beta;
-#pragma unroll
-      for (int q = 0; q < 3; q++) field[c + q] = alpha * fa[q] + beta * fb[q] + gamma * fe[q];
-    }
-    __syncthreads();
-  }
-}
-ESF_BOUNDS(kPassWave, kWaveThreads);
 
 // sweepVectorField's face copies, one axis per launch (z, then y, then x):
 // each thread copies both faces of its line in the reference's order
@@ -245,7 +491,7 @@ ESF_BOUNDS(kFaceCopy, 1024);
 
 template <class GridT>
 __device__ __forceinline__ void kFillFirst(const GridT& wg, int* first) {
-  if (threadIdx.x < 3) first[threadIdx.x] = INT_MAX;
+  if (threadIdx.x < 24) first[threadIdx.x] = INT_MAX;
 }
 ESF_BOUNDS(kFillFirst, 1024);
 
@@ -264,9 +510,33 @@ Sweep passRange(int i0, int i1, int j0, int j1, int k0, int k1) {
   return s;
 }
 
-// the context's sweep integers: three first-clear flags of a pass, or the
-// six extent counters of computeSDF
-constexpr int kSweepInts = 8;
+// the context's sweep integers: three first-clear flags of each of the eight
+// passes (or the six extent counters of computeSDF), then from kSyncInts on
+// the epoch and the tickets of kPencil
+constexpr int kSyncInts = 32;
+constexpr int kSweepInts = kSyncInts + 1 + kSweepTickets;
+
+// words of kPencil's edge buffer for sweeps of C doubles
+long edgeWords(int ni, int nj, int nk, int C) {
+  const long nJ = cdiv(nj, kRows), nK = cdiv(nk, kRows);
+  return ((nJ - 1) * nK + nJ * (nK - 1)) * ni * kRows * 2 * C;
+}
+// for the sweeps of a box (its last node along an axis is never one of them)
+long edgeWordsOf(const int box[6], int C) {
+  return edgeWords(box[3] - box[0] - 1, box[4] - box[1] - 1, box[5] - box[2] - 1, C);
+}
+
+int pencils(const Sweep& s) { return cdiv(s.nj, kRows) * cdiv(s.nk, kRows); }
+
+esf_status growEdges(esf_ctx* ctx, long words) {
+  esf_status st;
+  if (!ctx->swFirst && (st = devAlloc(ctx, &ctx->swFirst, kSweepInts))) return st;
+  if (words > ctx->swEdgeCap) {
+    if ((st = devAlloc(ctx, &ctx->swEdge, words))) return st;
+    ctx->swEdgeCap = words;
+  }
+  return ESF_OK;
+}
 
 esf_status checkBox(esf_ctx* ctx, const int box[6]) {
   const Dims& d = ctx->d;
@@ -279,7 +549,9 @@ esf_status checkBox(esf_ctx* ctx, const int box[6]) {
   return ESF_OK;
 }
 
-esf_status sweepPhiDevice(esf_ctx* ctx, const SweepBox& b, const double* mass, double* phi) {
+// one round of sweepPhi; ints, edge: kPencil's (slots 8 round .. 8 round + 7)
+esf_status sweepPhiDevice(esf_ctx* ctx, const SweepBox& b, const double* mass, double* phi,
+                          int round, int* ints, unsigned long long* edge) {
   for (int s = 0; s < 8; s++) {
     const int dx = (s & 2) ? -1 : 1, dy = (s & 1) ? -1 : 1, dz = (s & 4) ? -1 : 1;
     // ascending from min + 1 to max - 1, descending from max - 2 to min
@@ -293,7 +565,10 @@ esf_status sweepPhiDevice(esf_ctx* ctx, const SweepBox& b, const double* mass, d
     w.ni = b.x1 - b.x0 - 1;
     w.nj = b.y1 - b.y0 - 1;
     w.nk = b.z1 - b.z0 - 1;
-    launch<ESF_K(kPhiWave)>(ctx, dim3(1), dim3(kWaveThreads), b, w, mass, phi);
+    if (w.ni <= 0 || w.nj <= 0 || w.nk <= 0) continue;
+    launch<ESF_KT(kPencil, 1, true)>(ctx, dim3(pencils(w)), dim3(192), b, w, mass,
+                                     (const double2*)nullptr, phi,
+                                     SweepSync{ints, edge, 8 * round + s});
   }
   return hipGetLastError() == hipSuccess ? ESF_OK : ESF_ERR_DEVICE;
 }
@@ -305,9 +580,13 @@ esf_status sweepPhiRounds(esf_ctx* ctx, const int box[6], const double* mass, do
   const Dims& d = ctx->d;
   if (!(box[3] > box[0] && box[4] > box[1] && box[5] > box[2])) return ESF_OK;
   const SweepBox b{d.X, d.Y, d.Z, box[0], box[1], box[2], box[3], box[4], box[5]};
+  esf_status st = growEdges(ctx, edgeWordsOf(box, 1));
+  if (st) return st;
+  int* ints = ctx->swFirst + kSyncInts;
   for (int r = 0; r < rounds; r++) {
-    esf_status st = sweepPhiDevice(ctx, b, mass, phi);
-    if (st) return st;
+    const int slots = kSweepTickets / 8;
+    if (r % slots == 0) launch<ESF_K(kSweepStart)>(ctx, dim3(1), dim3(64), ints);
+    if ((st = sweepPhiDevice(ctx, b, mass, phi, r % slots, ints, ctx->swEdge))) return st;
   }
   return ESF_OK;
 }
@@ -319,17 +598,20 @@ esf_status extendDevice(esf_ctx* ctx, const int box[6], const double* m, const d
   esf_status st = checkBox(ctx, box);
   if (st) return st;
   const Dims& d = ctx->d;
-  const long boxNodes = (long)(box[3] - box[0]) * (box[4] - box[1]) * (box[5] - box[2]);
-  if (!ctx->swFirst && (st = devAlloc(ctx, &ctx->swFirst, kSweepInts))) return st;
-  if ((size_t)boxNodes > ctx->swCoefCap) {
-    if ((st = devAlloc(ctx, &ctx->swCoef, boxNodes))) return st;
-    ctx->swCoefCap = boxNodes;
+  // nodes of a pass: the box without its faces
+  const long cells =
+      (long)(box[3] - box[0] - 2) * (box[4] - box[1] - 2) * (box[5] - box[2] - 2);
+  if ((st = growEdges(ctx, edgeWordsOf(box, 3)))) return st;
+  if ((size_t)(8 * cells) > ctx->swCoefCap) {
+    if ((st = devAlloc(ctx, &ctx->swCoef, 8 * cells))) return st;
+    ctx->swCoefCap = 8 * cells;
   }
   const SweepBox b{d.X, d.Y, d.Z, box[0], box[1], box[2], box[3], box[4], box[5]};
   int* first = ctx->swFirst;
+  int* ints = first + kSyncInts;
   const int x0 = b.x0, y0 = b.y0, z0 = b.z0, x1 = b.x1, y1 = b.y1, z1 = b.z1;
   // sweepVectorField's eight passes (:524-545)
-  const Sweep passes[8] = {
+  const Passes passes = {{
       passRange(x0 + 1, x1 - 1, y0 + 1, y1 - 1, z0 + 1, z1 - 1),
       passRange(x0 + 1, x1 - 1, y1 - 2, y0, z0 + 1, z1 - 1),
       passRange(x1 - 2, x0, y0 + 1, y1 - 1, z0 + 1, z1 - 1),
@@ -337,19 +619,20 @@ esf_status extendDevice(esf_ctx* ctx, const int box[6], const double* m, const d
       passRange(x0 + 1, x1 - 1, y0 + 1, y1 - 1, z1 - 2, z0),
       passRange(x0 + 1, x1 - 1, y1 - 2, y0, z1 - 2, z0),
       passRange(x1 - 2, x0, y0 + 1, y1 - 1, z1 - 2, z0),
-      passRange(x1 - 2, x0, y1 - 2, y0, z1 - 2, z0)};
+      passRange(x1 - 2, x0, y1 - 2, y0, z1 - 2, z0)}};
+  // the flags and coefficients depend on phi and the mass, the same in all
+  // four rounds
+  launch<ESF_K(kFillFirst)>(ctx, dim3(1), dim3(64), first);
+  const int per = std::min(cdiv(cells, 256), 256);
+  launch<ESF_K(kPassFlags)>(ctx, dim3(8 * per), dim3(256), b, passes, per, m, ph, first);
+  launch<ESF_K(kPassCoef)>(ctx, dim3(8 * per), dim3(256), b, passes, per, m, ph,
+                           (const int*)first, ctx->swCoef);
+  launch<ESF_K(kSweepStart)>(ctx, dim3(1), dim3(64), ints);
   for (int round = 0; round < 4; round++) {
-    for (const Sweep& sw : passes) {
-      const long cells = (long)sw.ni * sw.nj * sw.nk;
-      if (cells == 0) continue;
-      launch<ESF_K(kFillFirst)>(ctx, dim3(1), dim3(64), first);
-      launch<ESF_K(kPassFlags)>(ctx, dim3(std::min<long>(cdiv(cells, 256), 2048)), dim3(256), b, sw,
-                                m, ph, first);
-      launch<ESF_K(kPassCoef)>(ctx, dim3(std::min<long>(cdiv(cells, 256), 2048)), dim3(256), b, sw,
-                               m, ph, (const int*)first, ctx->swCoef);
-      launch<ESF_K(kPassWave)>(ctx, dim3(1), dim3(kWaveThreads), b, sw, (const double2*)ctx->swCoef,
-                               f);
-    }
+    for (int p = 0; p < 8; p++)
+      launch<ESF_KT(kPencil, 3, false)>(ctx, dim3(pencils(passes.s[p])), dim3(192), b, passes.s[p],
+                                        m, (const double2*)(ctx->swCoef + p * cells), f,
+                                        SweepSync{ints, ctx->swEdge, 8 * round + p});
     // the faces: z (:547-552), y (:554-558), x (:560-564)
     const long lines[3] = {(long)(y1 - y0) * (z1 - z0), (long)(x1 - x0) * (z1 - z0),
                            (long)(x1 - x0) * (y1 - y0)};
@@ -375,32 +658,40 @@ esf_status sweepStaging(esf_ctx* ctx) {
 using namespace esf;
 
 // The allocation-free computeSDF's device memory (esf_compute_sdf_noalloc):
-// one array per GPU, resident while the process lives.  [0, 32) doubles hold
-// the extent counters, then the mass and phi of up to kSdfScratchNodes nodes
-// (the (128 + 1)^3 nodes of a 128^3-cell grid), 34.3 MB in all.  Host code
+// one array per GPU, resident while the process lives.  [0, 64) doubles hold
+// the extent counters and kPencil's integers, then the mass and phi of up to
+// kSdfScratchNodes nodes (the (128 + 1)^3 nodes of a 128^3-cell grid) and
+// kPencil's edge words for any box of such a grid, 45.5 MB in all.  Host code
 // never passes `scratch` itself to a kernel or a copy (on the host the name
 // is only a stand-in): it uses the device address hipGetSymbolAddress
 // returns, looked up once per device.
 constexpr long kSdfScratchNodes = 129L * 129 * 129;
-constexpr long kSdfScratchDoubles = 32 + 2 * kSdfScratchNodes;
+// kPencil's words: at most 0.64 per node over all shapes (rows of 9 x 9)
+constexpr long kSdfScratchEdges = kSdfScratchNodes * 13 / 20;
+constexpr long kSdfScratchHead = 64;  // doubles
+static_assert(2 * kSdfScratchHead >= kSweepInts, "the integers fit the head");
+constexpr long kSdfScratchDoubles = kSdfScratchHead + 2 * kSdfScratchNodes + kSdfScratchEdges;
 static __device__ __align__(256) double scratch[kSdfScratchDoubles];
 
 namespace esf {
 namespace {
 
-// the extent counters start at (X, Y, Z, 0, 0, 0): written by a kernel,
-// so the call works from memory the host cannot address
+// the extent counters start at (X, Y, Z, 0, 0, 0), kPencil's tickets at 0:
+// written by a kernel, so the call works from memory the host cannot address
 template <class GridT>
 __device__ __forceinline__ void kExtInit(const GridT& wg, int* ext, int X, int Y, int Z) {
   if (threadIdx.x < 6) ext[threadIdx.x] = threadIdx.x == 0 ? X : threadIdx.x == 1 ? Y
                                           : threadIdx.x == 2 ? Z : 0;
+  kSweepStart(wg, ext + kSyncInts);
 }
 ESF_BOUNDS(kExtInit, 1024);
 
 // computeSDF on the device buffers dm (the mass, n doubles), dphi (n
-// doubles) and dext (6 ints), all the caller's: boxes to the host, phi back
+// doubles), dext (kSweepInts ints) and edge (kPencil's words for the grid;
+// null: the context's, grown to the box), all the caller's: boxes to the
+// host, phi back
 esf_status computeSdfOn(esf_ctx* ctx, const double* mass, double* phi, int box[6], int tight[6],
-                        double* dm, double* dphi, int* dext) {
+                        double* dm, double* dphi, int* dext, unsigned long long* edge) {
   const Dims& d = ctx->d;
   const long n = d.nodes;
   ESF_HIP(hipMemcpyAsync(dm, mass, 8 * n, hipMemcpyHostToDevice, ctx->stream));
@@ -422,10 +713,14 @@ esf_status computeSdfOn(esf_ctx* ctx, const double* mass, double* phi, int box[6
   const bool sweep = box[3] > box[0] && box[4] > box[1] && box[5] > box[2];
   if (sweep) {
     const SweepBox b{d.X, d.Y, d.Z, box[0], box[1], box[2], box[3], box[4], box[5]};
-    for (int r = 0; r < 2; r++) {
-      esf_status st = sweepPhiDevice(ctx, b, dm, dphi);
-      if (st) return st;
+    esf_status st;
+    if (edge && edgeWordsOf(box, 1) > kSdfScratchEdges) return ESF_ERR_INVALID;
+    if (!edge) {
+      if ((st = growEdges(ctx, edgeWordsOf(box, 1)))) return st;
+      edge = ctx->swEdge;
     }
+    for (int r = 0; r < 2; r++)
+      if ((st = sweepPhiDevice(ctx, b, dm, dphi, r, dext + kSyncInts, edge))) return st;
   }
   ESF_HIP(hipMemcpyAsync(phi, dphi, 8 * n, hipMemcpyDeviceToHost, ctx->stream));
   ESF_HIP(streamSync(ctx));
@@ -475,7 +770,8 @@ esf_status esf_compute_sdf(esf_ctx* ctx, const double* mass, double* phi, int bo
   // staging held by the context (allocated on the first call)
   esf_status st = sweepStaging(ctx);
   if (st) return st;
-  return computeSdfOn(ctx, mass, phi, box, tight, ctx->swMass, ctx->swPhi, ctx->swFirst);
+  return computeSdfOn(ctx, mass, phi, box, tight, ctx->swMass, ctx->swPhi, ctx->swFirst,
+                      nullptr);
 }
 
 esf_status esf_compute_sdf_noalloc(esf_ctx* ctx, const double* mass, double* phi, int box[6],
@@ -490,8 +786,9 @@ esf_status esf_compute_sdf_noalloc(esf_ctx* ctx, const double* mass, double* phi
   double* base = nullptr;
   esf_status st = scratchOn(ctx, ctx->device, &base);
   if (st) return st;
-  return computeSdfOn(ctx, mass, phi, box, tight, base + 32, base + 32 + kSdfScratchNodes,
-                      (int*)base);
+  double* const dm = base + kSdfScratchHead;
+  return computeSdfOn(ctx, mass, phi, box, tight, dm, dm + kSdfScratchNodes, (int*)base,
+                      (unsigned long long*)(dm + 2 * kSdfScratchNodes));
 }
 
 esf_status esf_extend_vector_field(esf_ctx* ctx, const int box[6], const double* mass,

@@ -261,7 +261,7 @@ esf_status esf_compute_sdf(esf_ctx* ctx, const double* mass, double* phi, int bo
  * tight serving loops, harnesses that forbid hipMalloc).  The same results
  * as esf_compute_sdf, bitwise; its device staging (mass, phi) and extent
  * counters live in a static device array of the library, one per GPU, held
- * while the process lives: 34.3 MB, enough for grids of at most 129^3 =
+ * while the process lives: 45.5 MB, enough for grids of at most 129^3 =
  * 2,146,689 nodes (larger grids: ESF_ERR_INVALID).  Every call on a GPU
  * uses that GPU's one array, so calls that overlap on one GPU (from
  * several threads or contexts) race; calls in sequence are safe, each
