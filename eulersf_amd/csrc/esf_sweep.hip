@@ -113,7 +113,7 @@ __device__ __forceinline__ double solveDistance3(double p, double q, double r, d
 // for the edge words, both through rings in LDS, and the first only stores.
 // (One wave doing all three waits for its stores whenever it looks for an
 // edge word: 319 us per sweep of phi over the box of two balls at 96^3
-// cells, 173 us this way.  One workgroup walking the planes of the whole box
+// cells, 160 us this way.  One workgroup walking the planes of the whole box
 // with a barrier each took 2 us per plane, 540 us at 64^3 cells, where this
 // takes 111 us.)
 constexpr int kRows = 8;
@@ -150,6 +150,20 @@ __device__ __forceinline__ void ldsPublish(int* c, int v) {
   __hip_atomic_store(c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// The first word of row `row` at i' of a tile's edge, and the distance between
+// its words.  The eight rows are one step apart, so what one step reads (and
+// writes) of them shares a slot i' + row: with the field's six words per value
+// whole lines move, and the passes of an 80^3-cell call take 5.9 ms where
+// [i'][row][q] took 8.1; phi's two words measured 5 % better the plain way.
+template <int C>
+__device__ __forceinline__ long edgeAt(int i, int row, int ni) {
+  if (C == 1) return ((long)i * kRows + row) * 2;
+  const int t = i + row, slot = t < ni ? t : ni >= kRows ? t - ni : t % ni;
+  return (long)slot * 2 * C * kRows + row;
+}
+template <int C>
+constexpr int kEdgeStep = C == 1 ? 1 : kRows;
+
 template <int C, bool PHI, class GridT>
 __device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
                                         const double* __restrict__ mass,
@@ -170,8 +184,7 @@ __device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
   const unsigned long long tag = (unsigned long long)(unsigned)(sync.ints[0] + sync.slot) << 32;
   const int J = tile % nJ, K = tile / nJ;
   const long strideJ = (long)s.dj * b.X, strideK = (long)s.dk * b.X * b.Y;
-  // edge words: ni x 8 rows x C doubles of 2 words per tile with a next one
-  // along j', then the same along k'
+  // the edge words, per tile with a next one along j', then along k'
   const long perTile = (long)s.ni * kRows * 2 * C;
   const int fromJ = K * (nJ - 1) + J - 1, fromK = (nJ - 1) * nK + (K - 1) * nJ + J;
   const int steps = s.ni + 2 * (kRows - 1);
@@ -179,8 +192,8 @@ __device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
   if (role == 2) {
     // edge streams: 0..7 row j' - 1 of lanes (0, k), 8..15 row k' - 1 of lanes
     // (j, 0), from the tile before or, at the box's edge, from the field,
-    // where no node of this sweep lies; lane 16 u + stream looks at steps
-    // u and u + 4 beyond those handed on
+    // where no node of this sweep lies; lane 16 u + stream looks at
+    // step u beyond those handed on (four steps a look: eight took longer)
     const int str = lane & 15, u = lane >> 4;
     const bool forJ = str < kRows;
     const int q8 = str & 7, ej = forJ ? 0 : q8, ek = forJ ? q8 : 0;
@@ -190,7 +203,7 @@ __device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
     const long mAt = nodeAt(b, s.i0, s.j0 + s.dj * eJ, s.k0 + s.dk * eK) -
                      (forJ ? strideJ : strideK);
     const unsigned long long* const in =
-        sync.edge + (forJ ? perTile * fromJ : perTile * fromK) + 2 * C * q8;
+        sync.edge + (forJ ? perTile * fromJ : perTile * fromK);
     int p = 0;
     while (p < steps) {
       const int room = ldsCount(&cnt[2]) + kRing - p;
@@ -198,54 +211,42 @@ __device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
         __builtin_amdgcn_s_sleep(1);
         continue;
       }
-      unsigned long long w[2][2 * C];
-      bool ready[2];
+      const int i = p + u - q8;
+      const bool need = row && i >= 0 && i < s.ni;
+      unsigned long long w[2 * C];
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int i = p + u + 4 * h - q8;
-        const bool need = row && i >= 0 && i < s.ni;
+      for (int q = 0; q < 2 * C; q++) w[q] = tag;
+      if (need && mem) {
+        const long c = mAt + (long)s.di * i;
 #pragma unroll
-        for (int q = 0; q < 2 * C; q++) w[h][q] = tag;
-        if (need && mem) {
-          const long c = mAt + (long)s.di * i;
-#pragma unroll
-          for (int q = 0; q < C; q++) {
-            const double v = f[C * c + q];
-            w[h][2 * q] = tag | (unsigned)__double2loint(v);
-            w[h][2 * q + 1] = tag | (unsigned)__double2hiint(v);
-          }
-        } else if (need) {
-          const unsigned long long* e = in + (long)i * kRows * 2 * C;
-#pragma unroll
-          for (int q = 0; q < 2 * C; q++)
-            w[h][q] = __hip_atomic_load(e + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int q = 0; q < C; q++) {
+          const double v = f[C * c + q];
+          w[2 * q] = tag | (unsigned)__double2loint(v);
+          w[2 * q + 1] = tag | (unsigned)__double2hiint(v);
         }
-      }
+      } else if (need) {
+        const unsigned long long* e = in + edgeAt<C>(i, q8, s.ni);
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        ready[h] = true;
-#pragma unroll
-        for (int q = 0; q < 2 * C; q++) ready[h] = ready[h] && (w[h][q] >> 32) == (tag >> 32);
+        for (int q = 0; q < 2 * C; q++)
+          w[q] = __hip_atomic_load(e + q * kEdgeStep<C>, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
       }
+      bool ready = true;
+#pragma unroll
+      for (int q = 0; q < 2 * C; q++) ready = ready && (w[q] >> 32) == (tag >> 32);
       // the leading steps whose 16 streams are all there, as far as the ring
       // has room
-      const unsigned long long m0 = __ballot(ready[0]), m1 = __ballot(ready[1]);
+      const unsigned long long m = __ballot(ready);
       int n = 0;
-      for (int t = 0; t < 8; t++) {
-        const unsigned long long m = t < 4 ? m0 >> (16 * t) : m1 >> (16 * (t - 4));
-        if ((m & 0xffff) != 0xffff) break;
-        n = t + 1;
-      }
+      while (n < 4 && ((m >> (16 * n)) & 0xffff) == 0xffff) n++;
       n = min(n, room);
       if (n == 0) continue;
+      if (u < n) {
+        double* o = ering + (((p + u) & (kRing - 1)) * 16 + str) * C;
 #pragma unroll
-      for (int h = 0; h < 2; h++)
-        if (u + 4 * h < n) {
-          double* o = ering + (((p + u + 4 * h) & (kRing - 1)) * 16 + str) * C;
-#pragma unroll
-          for (int q = 0; q < C; q++)
-            o[q] = __hiloint2double((int)(unsigned)w[h][2 * q + 1], (int)(unsigned)w[h][2 * q]);
-        }
+        for (int q = 0; q < C; q++)
+          o[q] = __hiloint2double((int)(unsigned)w[2 * q + 1], (int)(unsigned)w[2 * q]);
+      }
       p += n;
       ldsPublish(&cnt[1], p);
     }
@@ -293,8 +294,8 @@ __device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
     return;
   }
 
-  unsigned long long* const outJ = sync.edge + perTile * (fromJ + 1) + 2 * C * k;
-  unsigned long long* const outK = sync.edge + perTile * (fromK + nJ) + 2 * C * j;
+  unsigned long long* const outJ = sync.edge + perTile * (fromJ + 1);
+  unsigned long long* const outK = sync.edge + perTile * (fromK + nJ);
   const bool giveJ = j == kRows - 1 && J + 1 < nJ && row;
   const bool giveK = k == kRows - 1 && K + 1 < nK && row;
   double last[C], cur[C];  // the values at i' - 1 and of the last step
@@ -341,18 +342,22 @@ __device__ __forceinline__ void kPencil(const GridT& wg, SweepBox b, Sweep s,
         cur[q] = nv[q];
       }
       if (giveJ || giveK) {
+        unsigned long long* const oJ = outJ + edgeAt<C>(i, k, s.ni);
+        unsigned long long* const oK = outK + edgeAt<C>(i, j, s.ni);
 #pragma unroll
         for (int q = 0; q < C; q++) {
           const unsigned long long lo = tag | (unsigned)__double2loint(nv[q]);
           const unsigned long long hi = tag | (unsigned)__double2hiint(nv[q]);
-          const long w = (long)i * kRows * 2 * C + 2 * q;
+          constexpr int d = kEdgeStep<C>;
           if (giveJ) {
-            __hip_atomic_store(outJ + w, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(outJ + w + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(oJ + 2 * q * d, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(oJ + (2 * q + 1) * d, hi, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
           }
           if (giveK) {
-            __hip_atomic_store(outK + w, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(outK + w + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(oK + 2 * q * d, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(oK + (2 * q + 1) * d, hi, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
           }
         }
       }
