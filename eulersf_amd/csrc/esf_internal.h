@@ -152,6 +152,7 @@ struct DevSolid {
   long nPart = 0, capPart = 0;
   double *pPos = nullptr, *pVel = nullptr;
   int *pBin = nullptr, *binItems = nullptr;
+  void* partRec = nullptr;  // the particles' records in the bins' order
 };
 
 // the mixed form's pressure preconditioner (esf_fastdiag.hip): per axis the
