@@ -272,6 +272,7 @@ esf_status esf_ctx_create(esf_ctx** out, const esf_grid* g, const esf_params* p)
   if (!st && mixed && fdFits(d)) st = fdCreate(ctx);
   if (!st) st = dalloc(ctx, &ctx->energyPart, cdiv(N, 256));
   if (!st) st = dalloc(ctx, &ctx->sc, 8);
+  if (!st) st = dalloc(ctx, &ctx->crDelta, 2);
   if (!st) st = dalloc(ctx, &ctx->dmisc, 16);
   if (!st) st = dalloc(ctx, &ctx->meshOut, 6 * kMaxSolids + 32);
   if (!st) st = growSolidDofs(ctx, 0);

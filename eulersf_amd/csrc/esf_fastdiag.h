@@ -30,21 +30,41 @@ struct PcgDir {
   double* rz;
 };
 
-// the sum of nb partials, in every thread of the block (256 threads) and
-// bitwise the same in every block; lds: 4 doubles
-__device__ inline double blockTotal(int nb, const double* __restrict__ parts, double* lds) {
-  double a[4] = {0, 0, 0, 0};
-  for (int i = threadIdx.x; i < nb; i += 4 * 256) {
+// the sums of K sets of nb partials ([k nb + i]), in every thread of the block
+// (256 threads) and bitwise the same in every block; lds: 4 K doubles
+template <int K>
+__device__ inline void blockTotals(int nb, const double* __restrict__ parts, double* lds,
+                                   double (&t)[K]) {
+  double a[K];
 #pragma unroll
-    for (int u = 0; u < 4; u++) a[u] += i + 256 * u < nb ? parts[i + 256 * u] : 0.0;
+  for (int k = 0; k < K; k++) a[k] = 0;
+  for (int i = threadIdx.x; i < nb; i += 4 * 256) {
+    double v[K][4];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        v[k][u] = i + 256 * u < nb ? parts[(long)k * nb + i + 256 * u] : 0.0;
+#pragma unroll
+    for (int k = 0; k < K; k++) a[k] += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
   }
-  const double w = waveSum((a[0] + a[1]) + (a[2] + a[3]));
+  double w[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) w[k] = waveSum(a[k]);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < K; k++) lds[4 * k + (threadIdx.x >> 6)] = w[k];
   __syncthreads();
-  const double s = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+#pragma unroll
+  for (int k = 0; k < K; k++)
+    t[k] = (lds[4 * k] + lds[4 * k + 1]) + (lds[4 * k + 2] + lds[4 * k + 3]);
   __syncthreads();
-  return s;
+}
+__device__ inline double blockTotal(int nb, const double* __restrict__ parts, double* lds) {
+  double t[1];
+  blockTotals<1>(nb, parts, lds, t);
+  return t[0];
 }
 
 FdGeom fdGeom(const Dims& d);
@@ -60,6 +80,7 @@ void fdTest(esf_ctx* ctx, int it, double eps, CrScalars* hostOut);
 
 // esf_pressure.hip
 int spmvBlocks(const esf_ctx* ctx);
+int spmvPcgBlocks(const esf_ctx* ctx);
 esf_status spmvPcg(esf_ctx* ctx, const double* pOld, const float* z, double* pNew, double* q,
                    CrScalars* sc, const PcgDir& dir, double* parts);
 

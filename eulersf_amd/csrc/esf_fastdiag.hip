@@ -516,7 +516,7 @@ esf_status fdIteration(esf_ctx* ctx, int it, double eps) {
   esf_status st = spmvPcg(ctx, pOld, z, pNew, ctx->Ap, sc, dir, partsQ);
   if (st) return st;
   launch<ESF_K(kPcgUpdate)>(ctx, dim3(f.nbR), dim3(256), g, ctx->d.cells, (const double*)pNew,
-                            (const double*)ctx->Ap, ctx->lambda, ctx->r, f.r32, nbQ,
+                            (const double*)ctx->Ap, ctx->lambda, ctx->r, f.r32, spmvPcgBlocks(ctx),
                             (const double*)partsQ, (const double*)(f.rz + (it & 1)), sc, partsR);
   return hipGetLastError() == hipSuccess ? ESF_OK : ESF_ERR_DEVICE;
 }

@@ -270,6 +270,8 @@ struct esf_ctx {
   // pressure SpMV launch shape (fixed at creation): cell layers per block,
   // load sets in flight for the CR update and for the other modes
   int spmvLayers = 16, spmvLayersWide = 8, spmvDepthUpdate = 1, spmvDepthOther = 2;
+  bool spmvFlat = true;      // small grids take the flat kernel
+  double* crDelta = nullptr; // r . s of the pressure CR's last two iterations
   // device allocations held by the context (admission control of served scenes)
   std::unordered_map<void*, size_t> allocs;
   size_t deviceBytes = 0;

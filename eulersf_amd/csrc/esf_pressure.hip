@@ -65,6 +65,7 @@ struct SpmvArgs {
   int recursive;     // M_UPDATE: the finisher tests the recursive residual
   CrScalars* hostOut;  // M_CHECK (M_UPDATE when recursive): pinned slot for the scalar block
   PcgDir dir;        // M_PCG
+  double* delta;     // kSpmvFlat M_UPDATE: r . s of the last two iterations
   int px, pxy;       // M_PCG_RESID: the padded layout's strides
 };
 
@@ -489,6 +490,213 @@ __device__ __forceinline__ void kSpmv(const GridT& wg, Dims d, SpmvArgs<T> a, in
 }
 ESF_BOUNDS(kSpmv, 256);
 
+// The same products and updates for grids of few tiles, where the march above
+// is a chain of load latencies (33^3: 10 layers of it, 11.5 us, for 36 000
+// cells): a block owns FX x FY x FZ cells, issues every load it needs at once,
+// and runs the stages through LDS with one barrier each.  The halo makes it
+// load each operand 2.1 times, so past kFlatBlocks tiles the march is ahead.
+// The sums over cells and nodes keep the march's order.
+// The CR update also takes over its finisher: the first thing it needs is the
+// totals of the iteration before, which every block adds up itself from the
+// (double-buffered) partials, in one order, instead of a one-block kernel
+// between the updates (3.7 us).
+constexpr int FX = 16, FY = 8, FZ = 4;
+constexpr int FHX = FX + 2, FHY = FY + 2, FHZ = FZ + 2, FHALO = FHX * FHY * FHZ;
+constexpr int FNX = FX + 1, FNY = FY + 1, FNZ = FZ + 1, FNODES = FNX * FNY * FNZ;
+constexpr int FCELLS = FX * FY * FZ;
+constexpr int FHPT = (FHALO + 255) / 256, FNPT = (FNODES + 255) / 256, FCPT = FCELLS / 256;
+
+template <int MODE, class GridT>
+__device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<double> a, int tilesX,
+                                          int tilesY) {
+  if (a.sc && a.sc->done) return;
+  __shared__ double xs[FHALO];
+  __shared__ double ws[3][FNODES];
+  __shared__ double red[5 * 4];
+  const int tile = wg.block();
+  const int x0 = FX * (tile % tilesX), y0 = FY * ((tile / tilesX) % tilesY),
+            z0 = FZ * (tile / (tilesX * tilesY));
+
+  // every load of the block, addresses clamped into the grid
+  double hin[FHPT], hap[FHPT], hs[FHPT], hd[FHPT];
+  float he[FHPT];
+#pragma unroll
+  for (int u = 0; u < FHPT; u++) {
+    const int h = threadIdx.x + 256 * u;
+    const int hx = h % FHX, hy = (h / FHX) % FHY, hz = h / (FHX * FHY);
+    const int gx = min(max(x0 + hx - 1, 0), d.CX - 1), gy = min(max(y0 + hy - 1, 0), d.CY - 1),
+              gz = min(max(z0 + hz - 1, 0), d.CZ - 1);
+    const long c = gx + (long)gy * d.CX + gz * d.cslab;
+    hin[u] = a.in[c];
+    if (MODE == M_UPDATE) {
+      hap[u] = a.Ap[c];
+      hs[u] = a.s[c];
+      hd[u] = a.Dinv[c];
+    }
+    if (MODE == M_PCG) he[u] = a.e32[c];
+  }
+  double mi[FNPT];
+#pragma unroll
+  for (int u = 0; u < FNPT; u++) {
+    const int n = threadIdx.x + 256 * u;
+    const int i = x0 + n % FNX, j = y0 + (n / FNX) % FNY, k = z0 + n / (FNX * FNY);
+    mi[u] = a.minv[min(max(i, 1), d.X - 2) + (long)min(max(j, 1), d.Y - 2) * d.X +
+                   min(max(k, 1), d.Z - 2) * d.slab];
+  }
+  long oc[FCPT];
+  bool own[FCPT];
+  double oB[FCPT], oX[FCPT], oP[FCPT], oR[FCPT], oAp[FCPT], oS[FCPT], oD[FCPT];
+#pragma unroll
+  for (int u = 0; u < FCPT; u++) {
+    const int t = threadIdx.x + 256 * u;
+    const int cx = x0 + t % FX, cy = y0 + (t / FX) % FY, cz = z0 + t / (FX * FY);
+    own[u] = cx < d.CX && cy < d.CY && cz < d.CZ;
+    oc[u] = min(cx, d.CX - 1) + (long)min(cy, d.CY - 1) * d.CX + min(cz, d.CZ - 1) * d.cslab;
+    if (MODE == M_CHECK || MODE == M_PCG_RESID) oB[u] = a.b[oc[u]];
+    if (MODE == M_UPDATE) {
+      oX[u] = a.x[oc[u]];
+      oP[u] = a.p[oc[u]];
+      oR[u] = a.in[oc[u]];
+      oAp[u] = a.Ap[oc[u]];
+      oS[u] = a.s[oc[u]];
+      oD[u] = a.Dinv[oc[u]];
+    }
+  }
+
+  double alpha = 0, beta = 0;
+  if (MODE == M_UPDATE) {
+    // r.s, s.D^-1 s, Ap.D^-1 s, Ap.D^-1 Ap of the iteration before: kFinish's
+    // F_CR; the setup's finisher left the first iteration's in the block
+    double dNew = a.sc->delta;
+    if (a.iter > 0) {
+      const double* parts = a.partials + (1 + ((a.iter + 1) & 1) * 4) * (long)wg.blocks();
+      double t[4];
+      blockTotals<4>(wg.blocks(), parts, red, t);
+      const double delta = a.delta[(a.iter + 1) & 1];
+      dNew = t[0];
+      beta = dNew / delta;
+      const double apq = (t[1] + (2.0 * beta) * t[2]) + (beta * beta) * t[3];
+      alpha = (fabs(apq) > 0.0) ? dNew / apq : apq;
+    } else {
+      alpha = a.sc->alpha;
+      beta = a.sc->beta;
+    }
+    if (wg.block() == 0 && threadIdx.x == 0) a.delta[a.iter & 1] = dNew;
+  }
+  if (MODE == M_PCG) {
+    const double rz = blockTotal(a.dir.nb, a.dir.parts, red);
+    const int now = a.dir.iter & 1;
+    if (a.dir.iter > 0) beta = rz / a.dir.rz[1 - now];
+    if (wg.block() == 0 && threadIdx.x == 0) a.dir.rz[now] = rz;
+  }
+
+#pragma unroll
+  for (int u = 0; u < FHPT; u++) {
+    const int h = threadIdx.x + 256 * u;
+    if (h < FHALO) {
+      const int hx = h % FHX, hy = (h / FHX) % FHY, hz = h / (FHX * FHY);
+      const int gx = x0 + hx - 1, gy = y0 + hy - 1, gz = z0 + hz - 1;
+      double v = hin[u];
+      if (MODE == M_UPDATE) {
+        const double apn = hap[u] * beta + hs[u];
+        const double qq = apn * hd[u];
+        v = hin[u] - alpha * qq;
+      } else if (MODE == M_PCG) {
+        v = a.dir.iter > 0 ? (double)he[u] + beta * hin[u] : (double)he[u];
+      }
+      const bool in = gx >= 0 && gx < d.CX && gy >= 0 && gy < d.CY && gz >= 0 && gz < d.CZ;
+      xs[h] = in ? v : 0.0;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < FNPT; u++) {
+    const int n = threadIdx.x + 256 * u;
+    if (n < FNODES) {
+      const int nx = n % FNX, ny = (n / FNX) % FNY, nz = n / (FNX * FNY);
+      const double* L = xs + nx + FHX * (ny + FHY * nz);
+      double m0 = 0, m1 = 0, m2 = 0;
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const double v = L[(q & 1) + FHX * ((q >> 1) & 1) + FHX * FHY * (q >> 2)];
+        m0 += (q & 1) == 0 ? v : -v;
+        m1 += ((q >> 1) & 1) == 0 ? v : -v;
+        m2 += (q >> 2) == 0 ? v : -v;
+      }
+      const int i = x0 + nx, j = y0 + ny, k = z0 + nz;
+      const bool interior =
+          i >= 1 && i <= d.X - 2 && j >= 1 && j <= d.Y - 2 && k >= 1 && k <= d.Z - 2;
+      ws[0][n] = interior ? m0 * mi[u] : 0.0;
+      ws[1][n] = interior ? m1 * mi[u] : 0.0;
+      ws[2][n] = interior ? m2 * mi[u] : 0.0;
+    }
+  }
+  __syncthreads();
+  double part0 = 0, part1 = 0, part2 = 0, part3 = 0;
+#pragma unroll
+  for (int u = 0; u < FCPT; u++) {
+    const int t = threadIdx.x + 256 * u;
+    const int lx = t % FX, ly = (t / FX) % FY, lz = t / (FX * FY);
+    const int n0 = lx + FNX * (ly + FNY * lz);
+    double acc = 0;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int n = n0 + (q & 1) + FNX * ((q >> 1) & 1) + FNX * FNY * (q >> 2);
+      acc += (q & 1) ? ws[0][n] : -ws[0][n];
+      acc += ((q >> 1) & 1) ? ws[1][n] : -ws[1][n];
+      acc += (q >> 2) ? ws[2][n] : -ws[2][n];
+    }
+    if (own[u]) {
+      const long c = oc[u];
+      const double v = xs[lx + 1 + FHX * (ly + 1 + FHY * (lz + 1))];  // the cell's own input
+      if (MODE == M_UPDATE) {
+        const double apn = oAp[u] * beta + oS[u];
+        const double pn = oP[u] * beta + oR[u];
+        a.r[c] = v;
+        a.ApOut[c] = apn;
+        a.p[c] = pn;
+        a.x[c] = oX[u] + alpha * pn;
+        a.sOut[c] = acc;
+        const double sq = acc * oD[u];
+        part0 += v * acc;
+        part1 += acc * sq;
+        part2 += apn * sq;
+        part3 += apn * (apn * oD[u]);
+      } else if (MODE == M_CHECK) {
+        const double r = acc - oB[u];
+        part0 += r * r;
+      } else if (MODE == M_PCG) {
+        a.p[c] = v;
+        a.out[c] = acc;
+        part0 += v * acc;
+      } else if (MODE == M_PCG_RESID) {
+        const double rr = oB[u] - acc;
+        const int cx = x0 + lx, cy = y0 + ly, cz = z0 + lz;
+        a.r[c] = rr;
+        a.r32[(long)cz * a.pxy + cy * a.px + cx] = (float)rr;
+        part0 += rr * rr;
+        part1 += oB[u] * oB[u];
+      } else {
+        a.out[c] = acc;
+      }
+    }
+  }
+  if (MODE == M_APPLY) return;
+  if (MODE == M_UPDATE) {
+    double mine[4] = {part0, part1, part2, part3};
+    // (behind a check's set, which is written between two updates)
+    blockPartialsAt<4>(mine, a.partials + (1 + (a.iter & 1) * 4) * (long)wg.blocks(), red,
+                       wg.blocks(), wg.block());
+  } else if (MODE == M_PCG_RESID) {
+    double mine[2] = {part0, part1};
+    blockPartialsAt<2>(mine, a.partials, red, wg.blocks(), wg.block());
+  } else {
+    double mine[1] = {part0};
+    blockPartialsAt<1>(mine, a.partials, red, wg.blocks(), wg.block());
+  }
+}
+ESF_BOUNDS(kSpmvFlat, 256);
+
 // b = J v0 - c, c (boundary velocities), D = diag(S); also the FP32 copies
 // used by the mixed solve.  COUPLED_INTEGRATOR_3D.cpp:286-325 (c),
 // :694-709 (D, b).  D == nullptr: b and c only (the mixed step forms the
@@ -609,6 +817,8 @@ void spmvConfigure(esf_ctx* ctx) {
   const int forcedDepth = envInt("ESF_SPMV_DEPTH", 1, 3);
   ctx->spmvDepthUpdate = forcedDepth ? forcedDepth : 1;
   ctx->spmvDepthOther = forcedDepth ? forcedDepth : 2;
+  // a forced shape of the march is for the march
+  ctx->spmvFlat = !forcedLayers && !forcedDepth;
 }
 
 // `deep`: the FP64 CR update's shape
@@ -620,9 +830,33 @@ static void tileShape(const esf_ctx* ctx, bool deep, int& tx, int& ty, int& tz, 
   tz = cdiv(d.CZ, layers);
 }
 
+// tiles up to which the flat kernel is taken (its updates and checks also need
+// 9 partials a tile).  FLATMEAS
+constexpr int kFlatBlocks = 2048;
+static int flatBlocks(const Dims& d) {
+  const long nb = (long)cdiv(d.CX, FX) * cdiv(d.CY, FY) * cdiv(d.CZ, FZ);
+  return nb <= kFlatBlocks ? (int)nb : 0;
+}
+
 template <typename T, int MODE>
 esf_status launchSpmv(esf_ctx* ctx, const SpmvArgs<T>& a) {
   int tx, ty, tz, layers;
+  constexpr bool flat = sizeof(T) == 8 && (MODE == M_UPDATE || MODE == M_CHECK || MODE == M_PCG ||
+                                           MODE == M_PCG_RESID || MODE == M_APPLY);
+  if constexpr (flat) {
+    const Dims& d = ctx->d;
+    if (const int nb = ctx->spmvFlat ? flatBlocks(d) : 0) {
+      launchTimed<ESF_KT(kSpmvFlat, MODE)>(ctx, MODE > M_IR_RESID ? -1 : MODE, dim3(nb), dim3(256),
+                                           d, a, cdiv(d.CX, FX), cdiv(d.CY, FY));
+      if constexpr (MODE == M_CHECK)
+        launchFinish<F_CHECK, 1>(ctx, nb, a.sc, a.iter, 0, nullptr, a.hostOut);
+      if constexpr (MODE == M_PCG_RESID)
+        launchFinish<F_IR, 2>(ctx, nb, a.sc, 0, a.first, nullptr, a.hostOut);
+      if (hipGetLastError() == hipSuccess) return ESF_OK;
+      ctx->err = "kSpmvFlat launch";
+      return ESF_ERR_DEVICE;
+    }
+  }
   tileShape(ctx, sizeof(T) == 8 && MODE == M_UPDATE, tx, ty, tz, layers);
   const int nb = tx * ty * tz;
   const int depth = MODE == M_UPDATE ? ctx->spmvDepthUpdate : ctx->spmvDepthOther;
@@ -653,9 +887,18 @@ esf_status launchSpmv(esf_ctx* ctx, const SpmvArgs<T>& a) {
   return ESF_OK;
 }
 
+// the blocks of M_PCG's launch
+int spmvPcgBlocks(const esf_ctx* ctx) {
+  const int nb = ctx->spmvFlat ? flatBlocks(ctx->d) : 0;
+  if (nb) return nb;
+  int tx, ty, tz, layers;
+  tileShape(ctx, false, tx, ty, tz, layers);
+  return tx * ty * tz;
+}
+
 // the most blocks a launch takes (the partials buffer's size)
 int spmvBlocks(const esf_ctx* ctx) {
-  int nb = 0;
+  int nb = 2 * flatBlocks(ctx->d);  // two sets of partials
   for (bool deep : {true, false}) {
     int tx, ty, tz, layers;
     tileShape(ctx, deep, tx, ty, tz, layers);
@@ -830,6 +1073,7 @@ esf_status crSolve(esf_ctx* ctx, int which, const T* minv, const T* b, const T* 
   a.Ap = Ap;
   a.sc = &ctx->sc[which];
   a.partials = ctx->partials;
+  a.delta = ctx->crDelta;
   T* rA = r;
   T* rB = r2;
   a.in = x;
