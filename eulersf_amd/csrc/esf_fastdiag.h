@@ -31,20 +31,21 @@ struct PcgDir {
 };
 
 // the sums of K sets of nb partials ([k nb + i]), in every thread of the block
-// (256 threads) and bitwise the same in every block; lds: 4 K doubles
-template <int K>
+// (NT threads) and bitwise the same in every block; lds: K doubles per wave
+template <int K, int NT = 256>
 __device__ inline void blockTotals(int nb, const double* __restrict__ parts, double* lds,
                                    double (&t)[K]) {
   double a[K];
 #pragma unroll
   for (int k = 0; k < K; k++) a[k] = 0;
-  for (int i = threadIdx.x; i < nb; i += 4 * 256) {
+  constexpr int nt = NT, nw = NT / 64;
+  for (int i = threadIdx.x; i < nb; i += 4 * nt) {
     double v[K][4];
 #pragma unroll
     for (int k = 0; k < K; k++)
 #pragma unroll
       for (int u = 0; u < 4; u++)
-        v[k][u] = i + 256 * u < nb ? parts[(long)k * nb + i + 256 * u] : 0.0;
+        v[k][u] = i + nt * u < nb ? parts[(long)k * nb + i + nt * u] : 0.0;
 #pragma unroll
     for (int k = 0; k < K; k++) a[k] += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
   }
@@ -54,16 +55,21 @@ __device__ inline void blockTotals(int nb, const double* __restrict__ parts, dou
   __syncthreads();
   if ((threadIdx.x & 63) == 0)
 #pragma unroll
-    for (int k = 0; k < K; k++) lds[4 * k + (threadIdx.x >> 6)] = w[k];
+    for (int k = 0; k < K; k++) lds[nw * k + (threadIdx.x >> 6)] = w[k];
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < K; k++)
-    t[k] = (lds[4 * k] + lds[4 * k + 1]) + (lds[4 * k + 2] + lds[4 * k + 3]);
+  for (int k = 0; k < K; k++) {
+    double r = 0;
+#pragma unroll
+    for (int v = 0; v < nw; v++) r += lds[nw * k + v];
+    t[k] = r;
+  }
   __syncthreads();
 }
+template <int NT = 256>
 __device__ inline double blockTotal(int nb, const double* __restrict__ parts, double* lds) {
   double t[1];
-  blockTotals<1>(nb, parts, lds, t);
+  blockTotals<1, NT>(nb, parts, lds, t);
   return t[0];
 }
 

@@ -504,15 +504,16 @@ constexpr int FX = 16, FY = 8, FZ = 4;
 constexpr int FHX = FX + 2, FHY = FY + 2, FHZ = FZ + 2, FHALO = FHX * FHY * FHZ;
 constexpr int FNX = FX + 1, FNY = FY + 1, FNZ = FZ + 1, FNODES = FNX * FNY * FNZ;
 constexpr int FCELLS = FX * FY * FZ;
-constexpr int FHPT = (FHALO + 255) / 256, FNPT = (FNODES + 255) / 256, FCPT = FCELLS / 256;
 
-template <int MODE, class GridT>
+// FT threads a block
+template <int MODE, int FT, class GridT>
 __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<double> a, int tilesX,
                                           int tilesY) {
-  if (a.sc && a.sc->done) return;
+  constexpr int FHPT = (FHALO + FT - 1) / FT, FNPT = (FNODES + FT - 1) / FT, FCPT = FCELLS / FT;
+  const bool done = a.sc && a.sc->done;  // looked at once the loads are out
   __shared__ double xs[FHALO];
   __shared__ double ws[3][FNODES];
-  __shared__ double red[5 * 4];
+  __shared__ double red[4 * (FT / 64)];
   const int tile = wg.block();
   const int x0 = FX * (tile % tilesX), y0 = FY * ((tile / tilesX) % tilesY),
             z0 = FZ * (tile / (tilesX * tilesY));
@@ -522,7 +523,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
   float he[FHPT];
 #pragma unroll
   for (int u = 0; u < FHPT; u++) {
-    const int h = threadIdx.x + 256 * u;
+    const int h = threadIdx.x + FT * u;
     const int hx = h % FHX, hy = (h / FHX) % FHY, hz = h / (FHX * FHY);
     const int gx = min(max(x0 + hx - 1, 0), d.CX - 1), gy = min(max(y0 + hy - 1, 0), d.CY - 1),
               gz = min(max(z0 + hz - 1, 0), d.CZ - 1);
@@ -538,7 +539,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
   double mi[FNPT];
 #pragma unroll
   for (int u = 0; u < FNPT; u++) {
-    const int n = threadIdx.x + 256 * u;
+    const int n = threadIdx.x + FT * u;
     const int i = x0 + n % FNX, j = y0 + (n / FNX) % FNY, k = z0 + n / (FNX * FNY);
     mi[u] = a.minv[min(max(i, 1), d.X - 2) + (long)min(max(j, 1), d.Y - 2) * d.X +
                    min(max(k, 1), d.Z - 2) * d.slab];
@@ -548,7 +549,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
   double oB[FCPT], oX[FCPT], oP[FCPT], oR[FCPT], oAp[FCPT], oS[FCPT], oD[FCPT];
 #pragma unroll
   for (int u = 0; u < FCPT; u++) {
-    const int t = threadIdx.x + 256 * u;
+    const int t = threadIdx.x + FT * u;
     const int cx = x0 + t % FX, cy = y0 + (t / FX) % FY, cz = z0 + t / (FX * FY);
     own[u] = cx < d.CX && cy < d.CY && cz < d.CZ;
     oc[u] = min(cx, d.CX - 1) + (long)min(cy, d.CY - 1) * d.CX + min(cz, d.CZ - 1) * d.cslab;
@@ -563,6 +564,10 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
     }
   }
 
+  const double deltaOld = MODE == M_UPDATE ? a.delta[(a.iter + 1) & 1] : 0.0;
+  asm volatile("" ::: "memory");
+  if (done) return;
+
   double alpha = 0, beta = 0;
   if (MODE == M_UPDATE) {
     // r.s, s.D^-1 s, Ap.D^-1 s, Ap.D^-1 Ap of the iteration before: kFinish's
@@ -571,10 +576,9 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
     if (a.iter > 0) {
       const double* parts = a.partials + (1 + ((a.iter + 1) & 1) * 4) * (long)wg.blocks();
       double t[4];
-      blockTotals<4>(wg.blocks(), parts, red, t);
-      const double delta = a.delta[(a.iter + 1) & 1];
+      blockTotals<4, FT>(wg.blocks(), parts, red, t);
       dNew = t[0];
-      beta = dNew / delta;
+      beta = dNew / deltaOld;
       const double apq = (t[1] + (2.0 * beta) * t[2]) + (beta * beta) * t[3];
       alpha = (fabs(apq) > 0.0) ? dNew / apq : apq;
     } else {
@@ -584,7 +588,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
     if (wg.block() == 0 && threadIdx.x == 0) a.delta[a.iter & 1] = dNew;
   }
   if (MODE == M_PCG) {
-    const double rz = blockTotal(a.dir.nb, a.dir.parts, red);
+    const double rz = blockTotal<FT>(a.dir.nb, a.dir.parts, red);
     const int now = a.dir.iter & 1;
     if (a.dir.iter > 0) beta = rz / a.dir.rz[1 - now];
     if (wg.block() == 0 && threadIdx.x == 0) a.dir.rz[now] = rz;
@@ -592,7 +596,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
 
 #pragma unroll
   for (int u = 0; u < FHPT; u++) {
-    const int h = threadIdx.x + 256 * u;
+    const int h = threadIdx.x + FT * u;
     if (h < FHALO) {
       const int hx = h % FHX, hy = (h / FHX) % FHY, hz = h / (FHX * FHY);
       const int gx = x0 + hx - 1, gy = y0 + hy - 1, gz = z0 + hz - 1;
@@ -611,7 +615,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < FNPT; u++) {
-    const int n = threadIdx.x + 256 * u;
+    const int n = threadIdx.x + FT * u;
     if (n < FNODES) {
       const int nx = n % FNX, ny = (n / FNX) % FNY, nz = n / (FNX * FNY);
       const double* L = xs + nx + FHX * (ny + FHY * nz);
@@ -635,7 +639,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
   double part0 = 0, part1 = 0, part2 = 0, part3 = 0;
 #pragma unroll
   for (int u = 0; u < FCPT; u++) {
-    const int t = threadIdx.x + 256 * u;
+    const int t = threadIdx.x + FT * u;
     const int lx = t % FX, ly = (t / FX) % FY, lz = t / (FX * FY);
     const int n0 = lx + FNX * (ly + FNY * lz);
     double acc = 0;
@@ -695,7 +699,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
     blockPartialsAt<1>(mine, a.partials, red, wg.blocks(), wg.block());
   }
 }
-ESF_BOUNDS(kSpmvFlat, 256);
+ESF_BOUNDS(kSpmvFlat, 512);
 
 // b = J v0 - c, c (boundary velocities), D = diag(S); also the FP32 copies
 // used by the mixed solve.  COUPLED_INTEGRATOR_3D.cpp:286-325 (c),
@@ -830,9 +834,13 @@ static void tileShape(const esf_ctx* ctx, bool deep, int& tx, int& ty, int& tz, 
   tz = cdiv(d.CZ, layers);
 }
 
-// tiles up to which the flat kernel is taken (its updates and checks also need
-// 9 partials a tile).  FLATMEAS
-constexpr int kFlatBlocks = 2048;
+// Tiles up to which the flat kernel is taken, and up to which with 512 threads
+// a block (its updates and checks need 9 partials a tile).  Measured, us per
+// FP64 CR iteration with its share of the checks: march / flat 256 / flat 512
+// threads at 16^3 16.4 / 9.5 / 8.6, 33^3 17.1 / 9.8 / 9.2, 48^3 (216 tiles)
+// 16.8 / 10.1 / 9.8, 64^3 (512) 17.6 / 12.7 / 13.6, 80^3 (1000) 24.1 / 21.8 /
+// 22.2, 96^3 (1728) 30.0 / 37.4 / -.
+constexpr int kFlatBlocks = 1024, kFlatWide = 256;
 static int flatBlocks(const Dims& d) {
   const long nb = (long)cdiv(d.CX, FX) * cdiv(d.CY, FY) * cdiv(d.CZ, FZ);
   return nb <= kFlatBlocks ? (int)nb : 0;
@@ -846,8 +854,13 @@ esf_status launchSpmv(esf_ctx* ctx, const SpmvArgs<T>& a) {
   if constexpr (flat) {
     const Dims& d = ctx->d;
     if (const int nb = ctx->spmvFlat ? flatBlocks(d) : 0) {
-      launchTimed<ESF_KT(kSpmvFlat, MODE)>(ctx, MODE > M_IR_RESID ? -1 : MODE, dim3(nb), dim3(256),
-                                           d, a, cdiv(d.CX, FX), cdiv(d.CY, FY));
+      const int cls = MODE > M_IR_RESID ? -1 : MODE;
+      if (nb <= kFlatWide)
+        launchTimed<ESF_KT(kSpmvFlat, MODE, 512)>(ctx, cls, dim3(nb), dim3(512), d, a,
+                                                  cdiv(d.CX, FX), cdiv(d.CY, FY));
+      else
+        launchTimed<ESF_KT(kSpmvFlat, MODE, 256)>(ctx, cls, dim3(nb), dim3(256), d, a,
+                                                  cdiv(d.CX, FX), cdiv(d.CY, FY));
       if constexpr (MODE == M_CHECK)
         launchFinish<F_CHECK, 1>(ctx, nb, a.sc, a.iter, 0, nullptr, a.hostOut);
       if constexpr (MODE == M_PCG_RESID)
