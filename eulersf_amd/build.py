@@ -40,6 +40,7 @@ SOURCES = [
     os.path.join(CSRC, "esf_batch.hip"),
     os.path.join(HOST, "esf_scene.cpp"),
     os.path.join(HOST, "esf_frames.cpp"),
+    os.path.join(HOST, "esf_transfer.cpp"),
 ]
 
 

@@ -196,6 +196,7 @@ esf_status esf_ctx_create(esf_ctx** out, const esf_grid* g, const esf_params* p)
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return ESF_ERR_DEVICE;
   esf_ctx* ctx = new esf_ctx();
+  transferContext(1);
   hipGetDevice(&ctx->device);
   // ESF_TIGHT_LISTS=1 (tests): the solid DOF and valid-cell lists are
   // sized to exactly their last counts, so a step whose count rises takes
@@ -226,6 +227,7 @@ esf_status esf_ctx_create(esf_ctx** out, const esf_grid* g, const esf_params* p)
   ctx->defaultDt = p->dt;
   ctx->dt = p->dt;
   if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
+    transferContext(-1);
     delete ctx;
     return ESF_ERR_DEVICE;
   }
@@ -315,6 +317,7 @@ void esf_ctx_destroy(esf_ctx* ctx) {
   if (ctx->side) hipStreamDestroy(ctx->side);
   hipStreamDestroy(ctx->stream);
   delete ctx;
+  transferContext(-1);
 }
 
 const char* esf_last_error(const esf_ctx* ctx) { return ctx ? ctx->err.c_str() : "null context"; }
@@ -665,9 +668,7 @@ esf_status esf_download(esf_ctx* ctx, int field, int solid, void* dst, size_t by
     ctx->err = "download size " + std::to_string(bytes) + " != " + std::to_string(want);
     return ESF_ERR_INVALID;
   }
-  ESF_HIP(hipMemcpyAsync(dst, p, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  ESF_HIP(streamSync(ctx));
-  return ESF_OK;
+  return copyToHost(ctx, dst, p, bytes);
 }
 
 esf_status esf_compute_solid_mass(esf_ctx* ctx, int solid) {
@@ -1151,20 +1152,15 @@ esf_status esf_pressure_apply(esf_ctx* ctx, const double* x, double* y) {
   if (!ctx || !x || !y) return ESF_ERR_INVALID;
   const size_t bytes = 8 * ctx->d.cells;
   ESF_HIP(hipMemcpyAsync(ctx->r, x, bytes, hipMemcpyHostToDevice, ctx->stream));
-  esf_status st = pressureApplyDevice(ctx, ctx->r, ctx->s);
-  if (st) return st;
-  ESF_HIP(hipMemcpyAsync(y, ctx->s, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  ESF_HIP(streamSync(ctx));
-  return ESF_OK;
+  const esf_status st = pressureApplyDevice(ctx, ctx->r, ctx->s);
+  return st ? st : copyToHost(ctx, y, ctx->s, bytes);
 }
 
 esf_status esf_pressure_diag(esf_ctx* ctx, double* dOut) {
   if (!ctx || !dOut) return ESF_ERR_INVALID;
   esf_status st = pressureRhs(ctx);
   if (st) return st;
-  ESF_HIP(hipMemcpyAsync(dOut, ctx->D, 8 * ctx->d.cells, hipMemcpyDeviceToHost, ctx->stream));
-  ESF_HIP(streamSync(ctx));
-  return ESF_OK;
+  return copyToHost(ctx, dOut, ctx->D, 8 * ctx->d.cells);
 }
 
 esf_status esf_solid_apply(esf_ctx* ctx, const double* x, double* y) {
@@ -1193,8 +1189,7 @@ esf_status esf_pressure_solve(esf_ctx* ctx, const double* b, double* x, double e
   st = crSolve<double>(ctx, 0, ctx->minv, ctx->b, ctx->D, ctx->Dinv, ctx->lambda, ctx->r,
                                   ctx->r2, ctx->pdir, ctx->s, ctx->s2, ctx->Ap, ctx->Ap2, eps, maxIt, 3);
   if (st) return st;
-  ESF_HIP(hipMemcpyAsync(x, ctx->lambda, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  ESF_HIP(streamSync(ctx));
+  if ((st = copyToHost(ctx, x, ctx->lambda, bytes))) return st;
   solveReport(ctx->hostSc[3], maxIt, &it, &conv, &rr);
   if (iters) *iters = it;
   if (relres) *relres = rr;

@@ -507,6 +507,12 @@ inline esf_status devAlloc(esf_ctx* ctx, T** p, size_t count) {
   return devAllocBytes(ctx, (void**)p, count * sizeof(T));
 }
 
+// esf_transfer.cpp: device memory into a host array, ordered behind the
+// context's queued work and over on return; and the count of live contexts
+// its pinned slots go by
+esf_status copyToHost(esf_ctx* ctx, void* dst, const void* src, size_t bytes);
+void transferContext(int change);
+
 // esf_sweep.hip: rounds of sweepPhi over box (xmin, ymin, zmin, xmax,
 // ymax, zmax) on device fields; extendVectorField (four rounds of
 // sweepVectorField) of a device node field over box

@@ -699,6 +699,8 @@ esf_status computeSdfOn(esf_ctx* ctx, const double* mass, double* phi, int box[6
                         double* dm, double* dphi, int* dext, unsigned long long* edge) {
   const Dims& d = ctx->d;
   const long n = d.nodes;
+  // (the entry point that allocates nothing leaves the pinned slots alone too)
+  const bool noalloc = edge != nullptr;
   ESF_HIP(hipMemcpyAsync(dm, mass, 8 * n, hipMemcpyHostToDevice, ctx->stream));
   launch<ESF_K(kExtInit)>(ctx, dim3(1), dim3(64), dext, d.X, d.Y, d.Z);
   launch<ESF_K(kSdfInit)>(ctx, dim3(std::min<long>(cdiv(n, 256), 4096)), dim3(256), n, d.X, d.Y,
@@ -727,6 +729,7 @@ esf_status computeSdfOn(esf_ctx* ctx, const double* mass, double* phi, int box[6
     for (int r = 0; r < 2; r++)
       if ((st = sweepPhiDevice(ctx, b, dm, dphi, r, dext + kSyncInts, edge))) return st;
   }
+  if (!noalloc) return copyToHost(ctx, phi, dphi, 8 * n);
   ESF_HIP(hipMemcpyAsync(phi, dphi, 8 * n, hipMemcpyDeviceToHost, ctx->stream));
   ESF_HIP(streamSync(ctx));
   return ESF_OK;
@@ -808,7 +811,5 @@ esf_status esf_extend_vector_field(esf_ctx* ctx, const int box[6], const double*
   ESF_HIP(hipMemcpyAsync(ctx->swPhi, phi, 8 * n, hipMemcpyHostToDevice, ctx->stream));
   ESF_HIP(hipMemcpyAsync(ctx->swField, field, 24 * n, hipMemcpyHostToDevice, ctx->stream));
   if ((st = extendDevice(ctx, box, ctx->swMass, ctx->swPhi, ctx->swField))) return st;
-  ESF_HIP(hipMemcpyAsync(field, ctx->swField, 24 * n, hipMemcpyDeviceToHost, ctx->stream));
-  ESF_HIP(streamSync(ctx));
-  return hipGetLastError() == hipSuccess ? ESF_OK : ESF_ERR_DEVICE;
+  return copyToHost(ctx, field, ctx->swField, 24 * n);
 }
