@@ -122,8 +122,8 @@ esf_status growSolidDofs(esf_ctx* ctx, int need) {
   ctx->inboxSolids = std::max<int>(1, (int)ctx->solids.size());
   if ((st = dalloc(ctx, &ctx->inbox, 24 * cap * ctx->inboxSolids))) return st;
   if ((st = dalloc(ctx, &ctx->inboxX, 24 * cap * ctx->inboxSolids))) return st;
-  // 3 sets x 5 sums and a set of 4 x node-pass blocks (3 cap DOFs / 256)
-  if ((st = dalloc(ctx, &ctx->sPartials, 20 * (3 * cap / 256 + 1)))) return st;
+  // 3 sets x 5 sums and a set of 4 x node-pass blocks (at most 3 cap / 128 + 1)
+  if ((st = dalloc(ctx, &ctx->sPartials, 20 * (3 * cap / 128 + 1)))) return st;
   ctx->capSolid = (int)cap;
   return ESF_OK;
 }

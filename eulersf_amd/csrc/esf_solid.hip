@@ -313,25 +313,50 @@ __device__ inline double sumGroup(double v) {
   return v;
 }
 
-constexpr int kCellThreads = 256;  // cell-pass block (512 measured slower)
+constexpr int kCellThreads = 256;  // the largest cell-pass block (512 measured slower)
 
-template <int MODE, int LPC, class GridT>
-__device__ __forceinline__ void kSolidCell(const GridT& wg, Dims d, int nValid, int cap,
-                                           const int* __restrict__ cornerDof,
-                                           const double* __restrict__ cellMat,
+// the cells of every solid with any, each solid's in blocks of its own from
+// `start` on: one launch serves them all (three balls in a 101x58x75 box took
+// three launches of 6.1 us per iteration)
+struct CellBody {
+  int start, nValid, cap;
+  const int* cornerDof;
+  const double* cellMat;
+  double lambda, mu;
+  double *inbox, *inboxX;
+};
+// (room for three: a small argument record for the usual scenes)
+constexpr int kFewSolids = 3;
+template <int NB>
+struct CellBodies {
+  int n;
+  CellBody b[NB];
+};
+
+template <int MODE, int LPC, int NB, class GridT>
+__device__ __forceinline__ void kSolidCell(const GridT& wg, Dims d, CellBodies<NB> bodies,
                                            const double* __restrict__ in,
                                            const double* __restrict__ sd,
                                            const double* __restrict__ apd,
                                            const double* __restrict__ xin, const CrScalars* sc,
-                                           SolidPartials sp, double lambda, double mu,
-                                           double* __restrict__ inbox, double* __restrict__ inboxX) {
+                                           SolidPartials sp) {
 #pragma clang fp contract(on)
+  int body = 0;
+  for (int b = 1; b < bodies.n; b++)
+    if (wg.block() >= bodies.b[b].start) body = b;
+  const CellBody& cb = bodies.b[body];
+  const int nValid = cb.nValid, cap = cb.cap;
+  const int* __restrict__ cornerDof = cb.cornerDof;
+  const double* __restrict__ cellMat = cb.cellMat;
+  const double lambda = cb.lambda, mu = cb.mu;
+  double* __restrict__ inbox = cb.inbox;
+  double* __restrict__ inboxX = cb.inboxX;
   static_assert(LPC == 2 || LPC == 4 || LPC == 8, "lanes per cell");
   constexpr bool kCR = MODE != CELL_IN;   // the CR residual update at the corners
   constexpr bool kX = MODE == CELL_CRX;   // also K_e x
   constexpr int CPL = 8 / LPC;  // corners per lane
   __shared__ double grp[5 * kScalMaxGroups];
-  const int t = wg.block() * blockDim.x + threadIdx.x;
+  const int t = (wg.block() - cb.start) * blockDim.x + threadIdx.x;
   const int e = t / LPC, l = t % LPC;
   const bool live = e < nValid;
   // first round of loads, all unconditional (indices clamped in bounds,
@@ -696,46 +721,76 @@ static int cellLanes() {
   return lanes;
 }
 
-template <int MODE, int LPC>
+// A pass of fewer lanes than this leaves most CUs without a block of the full
+// size, while each of its waves keeps a CU's address units busy with some
+// forty gathers: smaller blocks spread it.  The 64^3 ball (3832 cells, 4781
+// nodes): cell pass 6.3 us in blocks of 256 threads, 5.1 in 64; node pass 5.1
+// in 512, 4.6 in 128.  At 128^3 (61 600 lanes, 103 000 DOFs) the large blocks
+// are as fast, with fewer partials to add up.
+constexpr long kSpreadLanes = 32768;
+
+template <int MODE, int LPC, int NB>
 static void cellPassLanes(esf_ctx* ctx, const double* in, const CrScalars* sc,
                           const SolidPartials& sp, const double* x) {
   const int cls = MODE == CELL_CR ? 14 : (MODE == CELL_CRX ? 16 : -1);
+  CellBodies<NB> bodies{};
+  long lanes = 0;
+  for (const DevSolid& so : ctx->solids) lanes += (long)LPC * so.nValid;
+  // (in a batched step the scenes fill the chip together, and only launches
+  // of one block size are merged; the results do not depend on it)
+  const int threads = !ctx->fiber && lanes < kSpreadLanes ? 64 : kCellThreads;
+  int blocks = 0;
   for (size_t b = 0; b < ctx->solids.size(); b++) {
-    DevSolid& so = ctx->solids[b];
-    if (so.nValid > 0) {
-      launchTimed<ESF_KT(kSolidCell, MODE, LPC)>(ctx, cls,
-                                                 dim3(cdiv((long)LPC * so.nValid, kCellThreads)),
-                                                 dim3(kCellThreads), ctx->d, so.nValid, so.capValid,
-                                                 (const int*)so.cornerDof,
-                                                 (const double*)so.cellMat, in,
-                                                 (const double*)ctx->sSd, (const double*)ctx->sApd,
-                                                 x, sc, sp, so.lambda, so.mu,
-                                                 ctx->inbox + 24L * ctx->capSolid * b,
-                                                 ctx->inboxX + 24L * ctx->capSolid * b);
-    }
+    const DevSolid& so = ctx->solids[b];
+    if (so.nValid <= 0) continue;
+    bodies.b[bodies.n++] = {blocks,
+                            so.nValid,
+                            so.capValid,
+                            so.cornerDof,
+                            so.cellMat,
+                            so.lambda,
+                            so.mu,
+                            ctx->inbox + 24L * ctx->capSolid * b,
+                            ctx->inboxX + 24L * ctx->capSolid * b};
+    blocks += cdiv((long)LPC * so.nValid, threads);
   }
+  if (!blocks) return;
+  launchTimed<ESF_KT(kSolidCell, MODE, LPC, NB)>(ctx, cls, dim3(blocks), dim3(threads), ctx->d, bodies,
+                                             in, (const double*)ctx->sSd,
+                                             (const double*)ctx->sApd, x, sc, sp);
 }
 
 template <int MODE>
 static void cellPass(esf_ctx* ctx, const double* in, const CrScalars* sc,
                      const SolidPartials& sp, const double* x = nullptr) {
   const int lanes = cellLanes();
+  const bool few = (int)ctx->solids.size() <= kFewSolids;
+  auto pass = [&](auto lpc) {
+    if (few)
+      cellPassLanes<MODE, lpc.value, kFewSolids>(ctx, in, sc, sp, x);
+    else
+      cellPassLanes<MODE, lpc.value, kMaxSolids>(ctx, in, sc, sp, x);
+  };
   if (lanes == 8)
-    cellPassLanes<MODE, 8>(ctx, in, sc, sp, x);
+    pass(std::integral_constant<int, 8>{});
   else if (lanes == 4)
-    cellPassLanes<MODE, 4>(ctx, in, sc, sp, x);
+    pass(std::integral_constant<int, 4>{});
   else
-    cellPassLanes<MODE, 2>(ctx, in, sc, sp, x);
+    pass(std::integral_constant<int, 2>{});
 }
 
+static int nodeThreads(const esf_ctx* ctx) {
+  return 3L * ctx->nSolid < kSpreadLanes ? 128 : kNodeThreads;
+}
 static int nodeBlocks(const esf_ctx* ctx) {
-  return cdiv(std::max(3L * ctx->nSolid, 1L), kNodeThreads);
+  return cdiv(std::max(3L * ctx->nSolid, 1L), nodeThreads(ctx));
 }
 
 template <int MODE>
 static void nodePass(esf_ctx* ctx, SolidNodeArgs& a) {
   launchTimed<ESF_KT(kSolidNode, MODE)>(ctx, MODE == S_CR ? 15 : (MODE == S_CRX ? 17 : -1),
-                                        dim3(nodeBlocks(ctx)), dim3(kNodeThreads), ctx->d, a);
+                                        dim3(nodeBlocks(ctx)), dim3(nodeThreads(ctx)), ctx->d,
+                                        a);
 }
 
 esf_status solidAdiag(esf_ctx* ctx) {
