@@ -155,6 +155,7 @@ struct DonePoller {
   double best = 0;
   bool stagnated = false;
   int stopIt = -1;  // stagnated: the last iteration the solve runs
+  int doneIter = -1;  // converged: the iteration whose check passed
   hipEvent_t own[kRing];  // the context's events for the marks
   hipEvent_t ev[kRing];   // the event marking each check (own[] alone)
   explicit DonePoller(esf_ctx* c, int w, bool stag = false, int lagIters = 2, int flatPolls = 4)
@@ -163,7 +164,10 @@ struct DonePoller {
   }
   bool seen(int ws) {
     const CrScalars& h = ctx->hostRing[ws];
-    if (h.done) return true;
+    if (h.done) {
+      doneIter = h.iter;
+      return true;
+    }
     if (!stagnation) return false;
     if (best == 0 || h.resnorm < best) {
       best = h.resnorm;

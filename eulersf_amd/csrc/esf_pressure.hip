@@ -39,6 +39,7 @@ enum SpmvMode {
   M_IR_RESID = 5,
   M_PCG = 6,        // p = z + beta p, q = S p, p . q (esf_fastdiag.hip)
   M_PCG_RESID = 7,  // r = b - S x, also in FP32 in the preconditioner's layout
+  M_UPDATE_CHECK = 8,  // kSpmvFlat: M_UPDATE and, in blocks of its own, M_CHECK
 };
 
 template <typename T>
@@ -65,7 +66,12 @@ struct SpmvArgs {
   int recursive;     // M_UPDATE: the finisher tests the recursive residual
   CrScalars* hostOut;  // M_CHECK (M_UPDATE when recursive): pinned slot for the scalar block
   PcgDir dir;        // M_PCG
-  double* delta;     // kSpmvFlat M_UPDATE: r . s of the last two iterations
+  // kSpmvFlat M_UPDATE: r . s of the last two iterations; the x it writes (x
+  // stays as it was for a check beside it); the iterate whose check rode
+  // with the update before (its verdict is this update's to find), or -1
+  double* delta;
+  T* xOut;
+  int verdict;
   int px, pxy;       // M_PCG_RESID: the padded layout's strides
 };
 
@@ -505,18 +511,20 @@ constexpr int FHX = FX + 2, FHY = FY + 2, FHZ = FZ + 2, FHALO = FHX * FHY * FHZ;
 constexpr int FNX = FX + 1, FNY = FY + 1, FNZ = FZ + 1, FNODES = FNX * FNY * FNZ;
 constexpr int FCELLS = FX * FY * FZ;
 
-// FT threads a block
+// The true-residual check of an iterate may ride beside the next update, in
+// blocks of its own (M_UPDATE_CHECK), and a later update finds the verdict: no
+// launch of the check's and of its finisher's (8.5 us at 33^3, every fifth
+// iteration) stands in the chain.
 template <int MODE, int FT, class GridT>
-__device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<double> a, int tilesX,
-                                          int tilesY) {
+__device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const SpmvArgs<double>& a,
+                                         int tilesX, int tilesY, double* xs, double (*ws)[FNODES],
+                                         double* red) {
   constexpr int FHPT = (FHALO + FT - 1) / FT, FNPT = (FNODES + FT - 1) / FT, FCPT = FCELLS / FT;
   const bool done = a.sc && a.sc->done;  // looked at once the loads are out
-  __shared__ double xs[FHALO];
-  __shared__ double ws[3][FNODES];
-  __shared__ double red[4 * (FT / 64)];
   const int tile = wg.block();
   const int x0 = FX * (tile % tilesX), y0 = FY * ((tile / tilesX) % tilesY),
             z0 = FZ * (tile / (tilesX * tilesY));
+  const double* in = MODE == M_CHECK ? a.x : a.in;
 
   // every load of the block, addresses clamped into the grid
   double hin[FHPT], hap[FHPT], hs[FHPT], hd[FHPT];
@@ -528,7 +536,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
     const int gx = min(max(x0 + hx - 1, 0), d.CX - 1), gy = min(max(y0 + hy - 1, 0), d.CY - 1),
               gz = min(max(z0 + hz - 1, 0), d.CZ - 1);
     const long c = gx + (long)gy * d.CX + gz * d.cslab;
-    hin[u] = a.in[c];
+    hin[u] = in[c];
     if (MODE == M_UPDATE) {
       hap[u] = a.Ap[c];
       hs[u] = a.s[c];
@@ -557,7 +565,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
     if (MODE == M_UPDATE) {
       oX[u] = a.x[oc[u]];
       oP[u] = a.p[oc[u]];
-      oR[u] = a.in[oc[u]];
+      oR[u] = in[oc[u]];
       oAp[u] = a.Ap[oc[u]];
       oS[u] = a.s[oc[u]];
       oD[u] = a.Dinv[oc[u]];
@@ -573,6 +581,20 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
     // r.s, s.D^-1 s, Ap.D^-1 s, Ap.D^-1 Ap of the iteration before: kFinish's
     // F_CR; the setup's finisher left the first iteration's in the block
     double dNew = a.sc->delta;
+    if (a.verdict >= 0) {
+      // kFinish's F_CHECK, by every block
+      const double rn = sqrt(blockTotal<FT>(wg.blocks(), a.partials, red));
+      const bool conv = rn < a.sc->eps * a.sc->bnorm;
+      if (wg.block() == 0 && threadIdx.x == 0) {
+        a.sc->resnorm = rn;
+        if (conv) {
+          a.sc->iter = a.verdict;
+          a.sc->done = 1;
+        }
+        if (a.hostOut) *a.hostOut = *a.sc;
+      }
+      if (conv) return;
+    }
     if (a.iter > 0) {
       const double* parts = a.partials + (1 + ((a.iter + 1) & 1) * 4) * (long)wg.blocks();
       double t[4];
@@ -659,7 +681,7 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
         a.r[c] = v;
         a.ApOut[c] = apn;
         a.p[c] = pn;
-        a.x[c] = oX[u] + alpha * pn;
+        a.xOut[c] = oX[u] + alpha * pn;
         a.sOut[c] = acc;
         const double sq = acc * oD[u];
         part0 += v * acc;
@@ -697,6 +719,24 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
   } else {
     double mine[1] = {part0};
     blockPartialsAt<1>(mine, a.partials, red, wg.blocks(), wg.block());
+  }
+}
+
+// FT threads a block
+template <int MODE, int FT, class GridT>
+__device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<double> a, int tilesX,
+                                          int tilesY) {
+  __shared__ double xs[FHALO];
+  __shared__ double ws[3][FNODES];
+  __shared__ double red[4 * (FT / 64)];
+  if constexpr (MODE == M_UPDATE_CHECK) {
+    const int nb = wg.blocks() / 2, b = wg.block();
+    if (b < nb)
+      spmvFlat<M_UPDATE, FT>(SceneGrid{b, nb}, d, a, tilesX, tilesY, xs, ws, red);
+    else
+      spmvFlat<M_CHECK, FT>(SceneGrid{b - nb, nb}, d, a, tilesX, tilesY, xs, ws, red);
+  } else {
+    spmvFlat<MODE, FT>(wg, d, a, tilesX, tilesY, xs, ws, red);
   }
 }
 ESF_BOUNDS(kSpmvFlat, 512);
@@ -840,34 +880,45 @@ static void tileShape(const esf_ctx* ctx, bool deep, int& tx, int& ty, int& tz, 
 // threads at 16^3 16.4 / 9.5 / 8.6, 33^3 17.1 / 9.8 / 9.2, 48^3 (216 tiles)
 // 16.8 / 10.1 / 9.8, 64^3 (512) 17.6 / 12.7 / 13.6, 80^3 (1000) 24.1 / 21.8 /
 // 22.2, 96^3 (1728) 30.0 / 37.4 / -.
-constexpr int kFlatBlocks = 1024, kFlatWide = 256;
+// A check beside an update shares its registers: at 33^3 (135 tiles) that is
+// the better way (8.8 us per iteration against 9.1), at 48^3 (216) neither, at
+// 64^3 the worse (14.3 against 13.2).
+constexpr int kFlatBlocks = 1024, kFlatWide = 256, kFlatRide = 160;
 static int flatBlocks(const Dims& d) {
   const long nb = (long)cdiv(d.CX, FX) * cdiv(d.CY, FY) * cdiv(d.CZ, FZ);
   return nb <= kFlatBlocks ? (int)nb : 0;
 }
 
+template <int MODE>
+static esf_status launchFlat(esf_ctx* ctx, int nb, const SpmvArgs<double>& a) {
+  const Dims& d = ctx->d;
+  const int cls = MODE == M_UPDATE_CHECK ? M_UPDATE : MODE > M_IR_RESID ? -1 : MODE;
+  const int blocks = MODE == M_UPDATE_CHECK ? 2 * nb : nb;
+  if (nb <= kFlatWide)
+    launchTimed<ESF_KT(kSpmvFlat, MODE, 512)>(ctx, cls, dim3(blocks), dim3(512), d, a,
+                                              cdiv(d.CX, FX), cdiv(d.CY, FY));
+  else
+    launchTimed<ESF_KT(kSpmvFlat, MODE, 256)>(ctx, cls, dim3(blocks), dim3(256), d, a,
+                                              cdiv(d.CX, FX), cdiv(d.CY, FY));
+  if (hipGetLastError() == hipSuccess) return ESF_OK;
+  ctx->err = "kSpmvFlat launch";
+  return ESF_ERR_DEVICE;
+}
+
 template <typename T, int MODE>
 esf_status launchSpmv(esf_ctx* ctx, const SpmvArgs<T>& a) {
   int tx, ty, tz, layers;
-  constexpr bool flat = sizeof(T) == 8 && (MODE == M_UPDATE || MODE == M_CHECK || MODE == M_PCG ||
+  // (the FP64 CR update's flat form is crFlat's)
+  constexpr bool flat = sizeof(T) == 8 && (MODE == M_CHECK || MODE == M_PCG ||
                                            MODE == M_PCG_RESID || MODE == M_APPLY);
   if constexpr (flat) {
-    const Dims& d = ctx->d;
-    if (const int nb = ctx->spmvFlat ? flatBlocks(d) : 0) {
-      const int cls = MODE > M_IR_RESID ? -1 : MODE;
-      if (nb <= kFlatWide)
-        launchTimed<ESF_KT(kSpmvFlat, MODE, 512)>(ctx, cls, dim3(nb), dim3(512), d, a,
-                                                  cdiv(d.CX, FX), cdiv(d.CY, FY));
-      else
-        launchTimed<ESF_KT(kSpmvFlat, MODE, 256)>(ctx, cls, dim3(nb), dim3(256), d, a,
-                                                  cdiv(d.CX, FX), cdiv(d.CY, FY));
+    if (const int nb = ctx->spmvFlat ? flatBlocks(ctx->d) : 0) {
+      const esf_status st = launchFlat<MODE>(ctx, nb, a);
       if constexpr (MODE == M_CHECK)
         launchFinish<F_CHECK, 1>(ctx, nb, a.sc, a.iter, 0, nullptr, a.hostOut);
       if constexpr (MODE == M_PCG_RESID)
         launchFinish<F_IR, 2>(ctx, nb, a.sc, 0, a.first, nullptr, a.hostOut);
-      if (hipGetLastError() == hipSuccess) return ESF_OK;
-      ctx->err = "kSpmvFlat launch";
-      return ESF_ERR_DEVICE;
+      return st;
     }
   }
   tileShape(ctx, sizeof(T) == 8 && MODE == M_UPDATE, tx, ty, tz, layers);
@@ -1055,6 +1106,77 @@ static esf_status waitSlot3(esf_ctx* ctx, CrScalars* out) {
   return ESF_OK;
 }
 
+// crSolve's loop on the flat kernel, after the set-up.  The verdict of a check
+// (every 5 iterations, CONJUGATE_RESIDUAL.inl:166-176) is found by the update
+// behind it, which leaves x alone when it passes.  On up to kFlatRide tiles the
+// check of iterate c rides beside update c + 1, which then writes x to the
+// other of the two lambda buffers (the other updates work in place), and
+// update c + 2 finds the verdict; on more it is a launch of its own before
+// update c + 1.  ctx->lambda is the accepted iterate's buffer on return.
+static esf_status crFlat(esf_ctx* ctx, int which, SpmvArgs<double> a, double* rA, double* rB,
+                         double* sA, double* sB, double* apA, double* apB, double* x, int maxIt,
+                         int slot, DonePoller& poll) {
+  const int nb = flatBlocks(ctx->d);
+  const bool ride = nb <= kFlatRide;
+  const int behind = ride ? 2 : 1;  // updates from an iterate to its verdict
+  double* xs[2] = {x, ctx->lambda2};
+  esf_status st = ESF_OK;
+  auto checked = [](int i) { return i > 0 && i % 5 == 0; };
+  auto check = [&](int i, double* xi) {  // the sums alone
+    a.iter = i;
+    a.in = a.x = xi;
+    return launchFlat<M_CHECK>(ctx, nb, a);
+  };
+  int n = 0;    // updates queued
+  int cur = 0;  // the buffer of the iterate after them
+  bool done = false;
+  while (n < maxIt && !done) {
+    const int i = n;
+    if (!ride && checked(i - 1) && (st = check(i - 1, xs[cur]))) return st;
+    a.iter = i;
+    a.in = rA;
+    a.r = rB;
+    a.s = sA;
+    a.sOut = sB;
+    a.Ap = apA;
+    a.ApOut = apB;
+    a.x = xs[cur];
+    if (ride && checked(i - 1)) cur ^= 1;
+    a.xOut = xs[cur];
+    a.verdict = checked(i - behind) ? i - behind : -1;
+    a.hostOut = a.verdict >= 0 ? poll.slot() : nullptr;
+    st = ride && checked(i - 1) ? launchFlat<M_UPDATE_CHECK>(ctx, nb, a)
+                                : launchFlat<M_UPDATE>(ctx, nb, a);
+    if (st) return st;
+    if (a.verdict >= 0) poll.mark(i);
+    std::swap(rA, rB);
+    std::swap(sA, sB);
+    std::swap(apA, apB);
+    n++;
+    done = poll.drain(i);
+  }
+  if (!done) {
+    // checks that no later update is there for: of iterate n - 2, made
+    // beside the last update, and of the last
+    if (ride && checked(n - 2)) launchFinish<F_CHECK, 1>(ctx, nb, a.sc, n - 2);
+    if (checked(n - 1)) {
+      if ((st = check(n - 1, xs[cur]))) return st;
+      launchFinish<F_CHECK, 1>(ctx, nb, a.sc, n - 1);
+    }
+  }
+  ctx->crQueued = n;
+  copyScalarsAsync(ctx, &ctx->sc[which], &ctx->hostSc[slot]);
+  int accepted = done ? poll.doneIter : -1;
+  if (!done) {
+    ESF_HIP(streamSync(ctx));
+    if (ctx->hostSc[slot].done) accepted = ctx->hostSc[slot].iter;
+  }
+  // iterate 5 m: the buffer before update 5 m + 1 moved on, m - 1 moves in
+  if (ride && accepted >= 0) cur = (accepted / 5 - 1) & 1;
+  if (cur) std::swap(ctx->lambda, ctx->lambda2);
+  return ESF_OK;
+}
+
 // CONJUGATE_RESIDUAL::solvePCR (matrix-free) on S, FP64 or FP32 vectors.
 // The update multiplies by Dinv = 1 / D where the reference divides by D
 // (JACOBI_PRECONDITIONER.h:35-37): the iterates differ from the
@@ -1122,6 +1244,10 @@ esf_status crSolve(esf_ctx* ctx, int which, const T* minv, const T* b, const T* 
     return e;
   };
   int i = 0;
+  if constexpr (sizeof(T) == 8) {
+    if (ctx->spmvFlat && flatBlocks(ctx->d))
+      return crFlat(ctx, which, a, rA, rB, sA, sB, apA, apB, x, maxIt, slot, poll);
+  }
   for (; i < maxIt; i++) {
     const bool read = recursive && i % kPollEvery == kPollEvery - 1;
     if ((st = update(i, read ? poll.slot() : nullptr))) return st;
@@ -1231,6 +1357,7 @@ static esf_status fdSolve(esf_ctx* ctx, double eps, int maxIt, CrScalars* h, int
       fdTest(ctx, it, eps, &ctx->hostSc[4]);
       SpmvArgs<double> a{};
       a.in = ctx->lambda;
+      a.x = ctx->lambda;
       a.minv = ctx->minv;
       a.b = ctx->b;
       a.sc = &ctx->sc[0];
