@@ -518,7 +518,7 @@ constexpr int FCELLS = FX * FY * FZ;
 template <int MODE, int FT, class GridT>
 __device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const SpmvArgs<double>& a,
                                          int tilesX, int tilesY, double* xs, double (*ws)[FNODES],
-                                         double* red) {
+                                         double (*os)[FCELLS], double* red) {
   constexpr int FHPT = (FHALO + FT - 1) / FT, FNPT = (FNODES + FT - 1) / FT, FCPT = FCELLS / FT;
   const bool done = a.sc && a.sc->done;  // looked at once the loads are out
   const int tile = wg.block();
@@ -554,7 +554,7 @@ __device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const S
   }
   long oc[FCPT];
   bool own[FCPT];
-  double oB[FCPT], oX[FCPT], oP[FCPT], oR[FCPT], oAp[FCPT], oS[FCPT], oD[FCPT];
+  double oB[FCPT], oX[FCPT], oP[FCPT];
 #pragma unroll
   for (int u = 0; u < FCPT; u++) {
     const int t = threadIdx.x + FT * u;
@@ -565,10 +565,6 @@ __device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const S
     if (MODE == M_UPDATE) {
       oX[u] = a.x[oc[u]];
       oP[u] = a.p[oc[u]];
-      oR[u] = in[oc[u]];
-      oAp[u] = a.Ap[oc[u]];
-      oS[u] = a.s[oc[u]];
-      oD[u] = a.Dinv[oc[u]];
     }
   }
 
@@ -627,6 +623,14 @@ __device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const S
         const double apn = hap[u] * beta + hs[u];
         const double qq = apn * hd[u];
         v = hin[u] - alpha * qq;
+        // the block's own cells' operands, for the cell stage
+        const int lx = hx - 1, ly = hy - 1, lz = hz - 1;
+        if (lx >= 0 && lx < FX && ly >= 0 && ly < FY && lz >= 0 && lz < FZ) {
+          const int t = lx + FX * (ly + FY * lz);
+          os[0][t] = apn;
+          os[1][t] = hd[u];
+          os[2][t] = hin[u];
+        }
       } else if (MODE == M_PCG) {
         v = a.dir.iter > 0 ? (double)he[u] + beta * hin[u] : (double)he[u];
       }
@@ -676,18 +680,18 @@ __device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const S
       const long c = oc[u];
       const double v = xs[lx + 1 + FHX * (ly + 1 + FHY * (lz + 1))];  // the cell's own input
       if (MODE == M_UPDATE) {
-        const double apn = oAp[u] * beta + oS[u];
-        const double pn = oP[u] * beta + oR[u];
+        const double apn = os[0][t], dinv = os[1][t];
+        const double pn = oP[u] * beta + os[2][t];
         a.r[c] = v;
         a.ApOut[c] = apn;
         a.p[c] = pn;
         a.xOut[c] = oX[u] + alpha * pn;
         a.sOut[c] = acc;
-        const double sq = acc * oD[u];
+        const double sq = acc * dinv;
         part0 += v * acc;
         part1 += acc * sq;
         part2 += apn * sq;
-        part3 += apn * (apn * oD[u]);
+        part3 += apn * (apn * dinv);
       } else if (MODE == M_CHECK) {
         const double r = acc - oB[u];
         part0 += r * r;
@@ -728,15 +732,18 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
                                           int tilesY) {
   __shared__ double xs[FHALO];
   __shared__ double ws[3][FNODES];
+  // M_UPDATE: Ap, 1 / D and the old r of the block's cells
+  constexpr bool upd = MODE == M_UPDATE || MODE == M_UPDATE_CHECK;
+  __shared__ double os[upd ? 3 : 1][FCELLS];
   __shared__ double red[4 * (FT / 64)];
   if constexpr (MODE == M_UPDATE_CHECK) {
     const int nb = wg.blocks() / 2, b = wg.block();
     if (b < nb)
-      spmvFlat<M_UPDATE, FT>(SceneGrid{b, nb}, d, a, tilesX, tilesY, xs, ws, red);
+      spmvFlat<M_UPDATE, FT>(SceneGrid{b, nb}, d, a, tilesX, tilesY, xs, ws, os, red);
     else
-      spmvFlat<M_CHECK, FT>(SceneGrid{b - nb, nb}, d, a, tilesX, tilesY, xs, ws, red);
+      spmvFlat<M_CHECK, FT>(SceneGrid{b - nb, nb}, d, a, tilesX, tilesY, xs, ws, os, red);
   } else {
-    spmvFlat<MODE, FT>(wg, d, a, tilesX, tilesY, xs, ws, red);
+    spmvFlat<MODE, FT>(wg, d, a, tilesX, tilesY, xs, ws, os, red);
   }
 }
 ESF_BOUNDS(kSpmvFlat, 512);
