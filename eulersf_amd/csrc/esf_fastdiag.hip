@@ -108,8 +108,18 @@ __device__ __forceinline__ void kFdXY(const GridT& wg, FdGeom g, const float* __
       if (wg.block() == 0 && threadIdx.x == 0) pcgReport(t, rr);
       return;
     }
-  } else if (wg.block() == 0 && threadIdx.x == 0) {
-    initScalarBlock(t.sc, 0);  // read by the later kernels only
+  } else {
+    // queued before the host has seen the first residual: nothing to do where
+    // that already passes (the block is read by the later kernels only)
+    const bool done = t.outer->done;
+    if (wg.block() == 0 && threadIdx.x == 0) {
+      initScalarBlock(t.sc, 0);
+      if (done) {
+        t.sc->iter = 0;
+        t.sc->done = 1;
+      }
+    }
+    if (done) return;
   }
   const int lane = threadIdx.x & 63, w = waveOf(), col = lane & 15, gr = lane >> 4;
   const int z = wg.block() / g.tx, kx0 = 32 * (wg.block() % g.tx);

@@ -24,6 +24,8 @@
 // ones), as r does.  A true-residual check every 5 iterations, as the
 // reference does.  Block partials are summed by a one-block finisher (fixed
 // order, deterministic).
+#include <limits>
+
 #include "esf_fastdiag.h"
 #include "esf_internal.h"
 #include "esf_krylov.h"
@@ -1338,7 +1340,8 @@ static esf_status fdResidual(esf_ctx* ctx, int first, CrScalars* hostOut) {
 
 // Conjugate gradients preconditioned by fast diagonalisation
 // (esf_fastdiag.hip) from lambda, whose residual fdResidual has formed.
-// *h: scalar block 0 as the last check of the true residual left it; *made
+// *h: scalar block 0 as the last check of the true residual left it (on
+// entry: not done, its residual infinite where the host has not looked); *made
 // iterations in *rounds starts.  It gives up (h->done == 0) past
 // kFdIterations, when the direction breaks down, or when a restart does not
 // halve the residual; lambda then holds the last iterate.
@@ -1408,7 +1411,12 @@ esf_status mixedSolve(esf_ctx* ctx, double eps, int maxIt, int* iters, bool* con
   bool residual = true;  // form the residual the refinement starts from
   if (ctx->fd.T) {
     if ((st = fdResidual(ctx, 1, &ctx->hostSc[3]))) return st;
-    if ((st = waitSlot3(ctx, &h))) return st;
+    // where the last solve needed iterations this one's are queued unseen
+    // (the wait leaves the device idle for some 20 us); a scene at rest, whose
+    // solves end here, waits instead
+    h.done = 0;
+    h.resnorm = std::numeric_limits<double>::infinity();
+    if (ctx->fd.last == 0 && (st = waitSlot3(ctx, &h))) return st;
     if (!h.done && (st = fdSolve(ctx, eps, maxIt, &h, &inner, &outer))) return st;
     residual = !h.done && inner < maxIt;
   }
