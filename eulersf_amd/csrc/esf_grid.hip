@@ -1463,7 +1463,7 @@ ESF_BOUNDS(kSolidVelocity, 1024);
 // advection
 // ---------------------------------------------------------------------------
 // Tiling of the solid-displacement advection: a block owns 32 x 8 nodes of
-// each layer and marches kSLZ layers in z; the interpolated field on the
+// each layer and marches `layers` layers in z; the interpolated field on the
 // tile plus a one-node halo sits in LDS for three consecutive layers (loaded
 // row by row, each row of the halo box one contiguous run), so the 8-corner
 // interpolations read LDS.  A point whose corners leave that window reads
@@ -1471,16 +1471,17 @@ ESF_BOUNDS(kSolidVelocity, 1024);
 // kernels stay one thread per node: tiled the same way they measured
 // slower, 137 vs 86 us and 66 vs 32 us at 128^3, their departure points
 // leaving the window more often.)
-constexpr int kSLX = 32, kSLY = 8, kSLZ = 8;
+constexpr int kSLX = 32, kSLY = 8;
 constexpr int kSLHX = kSLX + 2, kSLHY = kSLY + 2;
 constexpr int kSLLayer = kSLHX * kSLHY;  // halo nodes per layer
 static_assert(kSLX * kSLY == 256, "one node per thread and layer");
 
-__device__ inline void tileOf(int b, int tilesX, int tilesY, int& x0, int& y0, int& z0) {
+__device__ inline void tileOf(int b, int tilesX, int tilesY, int layers, int& x0, int& y0,
+                              int& z0) {
   const int tx = b % tilesX, ty = (b / tilesX) % tilesY, tz = b / (tilesX * tilesY);
   x0 = tx * kSLX;
   y0 = ty * kSLY;
-  z0 = tz * kSLZ;
+  z0 = tz * layers;
 }
 
 // advectFluidVelocityField  COUPLED_INTEGRATOR_3D.cpp:797-826
@@ -1554,11 +1555,12 @@ ESF_BOUNDS(kAdvectScalar, 256);
 template <class GridT>
 __device__ __forceinline__ void kSolidAdvectU(const GridT& wg, Dims d, const double* __restrict__ u,
                                               const double* __restrict__ sv, double dt,
-                                              double* __restrict__ unew, int tilesX, int tilesY) {
+                                              double* __restrict__ unew, int tilesX, int tilesY,
+                                              int layers) {
   __shared__ double w[3][3 * kSLLayer];
   int x0, y0, z0;
-  tileOf(wg.block(), tilesX, tilesY, x0, y0, z0);
-  const int zEnd = min(z0 + kSLZ, d.Z);
+  tileOf(wg.block(), tilesX, tilesY, layers, x0, y0, z0);
+  const int zEnd = min(z0 + layers, d.Z);
   // layer z of w into ring slot (z + 3) mod 3 (zeros outside the grid:
   // never read, the interpolation corners stay inside)
   auto loadLayer = [&](int z) {
@@ -1997,9 +1999,17 @@ esf_status solidCopyVelocity(esf_ctx* ctx) {
 
 esf_status solidFinalize(esf_ctx* ctx, double dt) {
   for (auto& so : ctx->solids) {
-    const int tX = cdiv(ctx->d.X, kSLX), tY = cdiv(ctx->d.Y, kSLY), tZ = cdiv(ctx->d.Z, kSLZ);
+    // a tile's march is one serial chain of layers, each a round of loads and
+    // two barriers: 8 layers (2 halo layers read for 8) where that leaves two
+    // tiles per CU, else as few as 2.  8 layers vs this rule, device time: 26
+    // vs 11 us at 17^3 nodes, 28 vs 15 us at 65^3 (2 layers), 37 vs 24 us at
+    // 102 x 59 x 76 (4), 42 vs 34 us for 12 scenes of 24-72 cells together
+    const int tX = cdiv(ctx->d.X, kSLX), tY = cdiv(ctx->d.Y, kSLY);
+    int layers = 8;
+    while (layers > 2 && tX * tY * cdiv(ctx->d.Z, layers) < 512) layers /= 2;
+    const int tZ = cdiv(ctx->d.Z, layers);
     launch<ESF_K(kSolidAdvectU)>(ctx, dim3(tX * tY * tZ), dim3(256), ctx->d, (const double*)so.u,
-                                 (const double*)so.vel, dt, so.unew, tX, tY);
+                                 (const double*)so.vel, dt, so.unew, tX, tY, layers);
     std::swap(so.u, so.unew);
     const Box& b = so.box;
     // the face extrapolation rides with X = x - u where the box is wide
