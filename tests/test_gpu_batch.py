@@ -158,3 +158,13 @@ def test_lists_grown_after_their_scan_same_bits(esf, monkeypatch):
     assert rises > 0
     check_batched(esf, texts, esf.ESF_MIXED, steps, usual)
     _say("tight lists: same bits batched")
+
+
+@pytest.mark.parametrize("count", [2, 20, 48])
+def test_batch_tables_in_the_argument_and_in_memory(esf, count):
+    """few scenes, whose tables every kernel takes as its argument, and as
+    many as need a table in device memory: both as alone"""
+    from eulersf_amd.serve import random_scene
+    texts = [random_scene(np.random.default_rng(100 + i), 12 + i % 5) for i in range(count)]
+    alone = run_alone(esf, texts, esf.ESF_MIXED, 2)
+    check_batched(esf, texts, esf.ESF_MIXED, 2, alone)
