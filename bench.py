@@ -10,7 +10,7 @@ A step is one esf_step: CFL, corotational stress, body forces, the three
 Schur-complement solves, solid finalize, mass gathering, advection of
 velocity and intensity, boundary conditions -- with all fields resident in
 HBM.  The scene runs twice: FP64 (the reference's CR, "plain") and mixed
-(FP32 CR inside FP64 iterative refinement).  `value` is the mixed form's
+(FP64 CG with an FP32 preconditioner).  `value` is the mixed form's
 steps/s; the FP64 rate, the speedup and the per-field difference between
 the two forms are reported beside it.
 
@@ -690,7 +690,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32 Krylov in f64 refinement (f64 elsewhere)",
+        "dtype": "f64 (f32 preconditioner in the mixed form's f64 CG)",
         "data": "synthetic scene (analytic sphere), no external data",
         "config": {"workload": f"unit-cube rubber ball, {n}^3 cells ({n + 1}^3 nodes), "
                                "sphere r=0.15 E=1e4 nu=0.3, rho 1000:1000, dt=1/240, "

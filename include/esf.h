@@ -253,7 +253,7 @@ esf_status esf_broad_phase(esf_ctx* ctx, double* alpha);
  * nodes widened by "extrapolation cells".  box and tight receive
  * {xmin, ymin, zmin, xmax, ymax, zmax} as _xmin.._zmax and _tightMin /
  * _tightMax ("tight border").  Bitwise the reference's sweeps, run on the
- * GPU plane by plane. */
+ * GPU by tiles of rows that march one step apart. */
 esf_status esf_compute_sdf(esf_ctx* ctx, const double* mass, double* phi, int box[6],
                            int tight[6]);
 /* esf_compute_sdf without allocating: no reference counterpart.  For
@@ -273,7 +273,7 @@ esf_status esf_compute_sdf_noalloc(esf_ctx* ctx, const double* mass, double* phi
  * the box faces) on a node field of 3 doubles per node, in place, where
  * mass == 0; phi and box as computeSDF leaves them.  The box must lie in
  * the grid and span at least 3 nodes per axis.  Bitwise the reference's
- * sweeps, run on the GPU plane by plane. */
+ * sweeps, run on the GPU by tiles of rows that march one step apart. */
 esf_status esf_extend_vector_field(esf_ctx* ctx, const int box[6], const double* mass,
                                    const double* phi, double* field);
 /* --- FLIP material particles (one solid per scene) ---------------------*/
