@@ -2003,10 +2003,11 @@ esf_status solidFinalize(esf_ctx* ctx, double dt) {
     // two barriers: 8 layers (2 halo layers read for 8) where that leaves two
     // tiles per CU, else as few as 2.  8 layers vs this rule, device time: 26
     // vs 11 us at 17^3 nodes, 28 vs 15 us at 65^3 (2 layers), 37 vs 24 us at
-    // 102 x 59 x 76 (4), 42 vs 34 us for 12 scenes of 24-72 cells together
+    // 102 x 59 x 76 (4).  A batch's scenes fill the chip together: 64 of them
+    // took 456 us per launch at 8 layers and 604 at 2 and 4 (12: 42 and 34)
     const int tX = cdiv(ctx->d.X, kSLX), tY = cdiv(ctx->d.Y, kSLY);
     int layers = 8;
-    while (layers > 2 && tX * tY * cdiv(ctx->d.Z, layers) < 512) layers /= 2;
+    while (!ctx->fiber && layers > 2 && tX * tY * cdiv(ctx->d.Z, layers) < 512) layers /= 2;
     const int tZ = cdiv(ctx->d.Z, layers);
     launch<ESF_K(kSolidAdvectU)>(ctx, dim3(tX * tY * tZ), dim3(256), ctx->d, (const double*)so.u,
                                  (const double*)so.vel, dt, so.unew, tX, tY, layers);
