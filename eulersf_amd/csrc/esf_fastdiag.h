@@ -73,6 +73,17 @@ __device__ inline double blockTotal(int nb, const double* __restrict__ parts, do
   return t[0];
 }
 
+// a solve's done flag for a launch in which a block sets it: the read of the
+// block's first thread, in all its threads.  Each wave reading for itself, a
+// block that starts while the flag is being set would have some waves leave
+// and the others add up LDS slots that nobody wrote.  (Blocks may differ: a
+// launch that sets the flag leaves the solve's vectors alone in every block.)
+__device__ inline bool blockDone(int done, int* lds) {
+  if (threadIdx.x == 0) *lds = done;
+  __syncthreads();
+  return *lds != 0;
+}
+
 FdGeom fdGeom(const Dims& d);
 // whether the preconditioner takes this grid
 bool fdFits(const Dims& d);

@@ -101,8 +101,9 @@ __device__ __forceinline__ void kFdXY(const GridT& wg, FdGeom g, const float* __
   constexpr int LD = 64 * MT + 4;
   __shared__ __align__(16) float L[32 * LD];
   __shared__ double red[4];
+  __shared__ int flag;
   if (t.iter > 0) {
-    if (t.sc->done) return;
+    if (blockDone(t.sc->done, &flag)) return;
     const double rr = blockTotal(t.nb, t.parts, red);
     if (pcgDone(t, rr)) {
       if (wg.block() == 0 && threadIdx.x == 0) pcgReport(t, rr);
@@ -372,7 +373,8 @@ __device__ __forceinline__ void kPcgUpdate(const GridT& wg, FdGeom g, long cells
                                            const double* __restrict__ rz, CrScalars* sc,
                                            double* parts) {
   __shared__ double red[4];
-  if (sc->done) return;
+  __shared__ int flag;
+  if (blockDone(sc->done, &flag)) return;
   const double pq = blockTotal(nbQ, partsQ, red);
   const bool ok = pq > 0.0;
   if (!ok && wg.block() == 0 && threadIdx.x == 0) sc->done = 2;

@@ -520,9 +520,9 @@ constexpr int FCELLS = FX * FY * FZ;
 template <int MODE, int FT, class GridT>
 __device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const SpmvArgs<double>& a,
                                          int tilesX, int tilesY, double* xs, double (*ws)[FNODES],
-                                         double (*os)[FCELLS], double* red) {
+                                         double (*os)[FCELLS], double* red, int* flag) {
   constexpr int FHPT = (FHALO + FT - 1) / FT, FNPT = (FNODES + FT - 1) / FT, FCPT = FCELLS / FT;
-  const bool done = a.sc && a.sc->done;  // looked at once the loads are out
+  bool done = a.sc && a.sc->done;  // looked at once the loads are out
   const int tile = wg.block();
   const int x0 = FX * (tile % tilesX), y0 = FY * ((tile / tilesX) % tilesY),
             z0 = FZ * (tile / (tilesX * tilesY));
@@ -572,6 +572,8 @@ __device__ __forceinline__ void spmvFlat(const GridT& wg, const Dims& d, const S
 
   const double deltaOld = MODE == M_UPDATE ? a.delta[(a.iter + 1) & 1] : 0.0;
   asm volatile("" ::: "memory");
+  // (a launch that finds a verdict may set the flag while its blocks read it)
+  if (MODE == M_UPDATE && a.verdict >= 0) done = blockDone(done, flag);
   if (done) return;
 
   double alpha = 0, beta = 0;
@@ -738,14 +740,15 @@ __device__ __forceinline__ void kSpmvFlat(const GridT& wg, Dims d, SpmvArgs<doub
   constexpr bool upd = MODE == M_UPDATE || MODE == M_UPDATE_CHECK;
   __shared__ double os[upd ? 3 : 1][FCELLS];
   __shared__ double red[4 * (FT / 64)];
+  __shared__ int flag;
   if constexpr (MODE == M_UPDATE_CHECK) {
     const int nb = wg.blocks() / 2, b = wg.block();
     if (b < nb)
-      spmvFlat<M_UPDATE, FT>(SceneGrid{b, nb}, d, a, tilesX, tilesY, xs, ws, os, red);
+      spmvFlat<M_UPDATE, FT>(SceneGrid{b, nb}, d, a, tilesX, tilesY, xs, ws, os, red, &flag);
     else
-      spmvFlat<M_CHECK, FT>(SceneGrid{b - nb, nb}, d, a, tilesX, tilesY, xs, ws, os, red);
+      spmvFlat<M_CHECK, FT>(SceneGrid{b - nb, nb}, d, a, tilesX, tilesY, xs, ws, os, red, &flag);
   } else {
-    spmvFlat<MODE, FT>(wg, d, a, tilesX, tilesY, xs, ws, os, red);
+    spmvFlat<MODE, FT>(wg, d, a, tilesX, tilesY, xs, ws, os, red, &flag);
   }
 }
 ESF_BOUNDS(kSpmvFlat, 512);
