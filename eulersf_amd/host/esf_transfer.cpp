@@ -67,7 +67,10 @@ void moveChunks(esf_ctx* ctx, char* host, const char* dev, size_t bytes, char* s
   auto check = [&](hipError_t e) {
     if (e != hipSuccess) failed->store((int)e);
   };
-  check(hipSetDevice(ctx->device));
+  // (worker 0 is the calling thread, whose current device is the caller's)
+  int was = ctx->device;
+  check(hipGetDevice(&was));
+  if (was != ctx->device) check(hipSetDevice(ctx->device));
   for (hipEvent_t& e : ev) check(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   size_t at[2] = {0, 0}, len[2] = {0, 0};
   int k = 0;
@@ -89,6 +92,7 @@ void moveChunks(esf_ctx* ctx, char* host, const char* dev, size_t bytes, char* s
   settle(k ^ 1);
   for (hipEvent_t e : ev)
     if (e) (void)hipEventDestroy(e);
+  if (was != ctx->device) (void)hipSetDevice(was);
 }
 
 }  // namespace
