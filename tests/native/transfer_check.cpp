@@ -127,5 +127,19 @@ int main(int argc, char** argv) {
     esf::transferContext(-1);
     report("end");
   }
+  if (!std::strcmp(what, "pinned")) {
+    // a destination the caller pinned, whole and from its middle
+    esf::transferContext(1);
+    copy(host.data(), dev.size());
+    report("pageable");
+    char* p = nullptr;
+    (void)hipHostMalloc((void**)&p, dev.size(), 0);
+    copy(p, dev.size());
+    report("pinned");
+    copy(p + 5 * MB, 4 * MB);
+    report("inside");
+    (void)hipHostFree(p);
+    esf::transferContext(-1);
+  }
   return 0;
 }

@@ -46,3 +46,11 @@ def test_the_callers_device_stays_current(check):
     assert s["large"]["chunks"] > 0 and s["large"]["device"] == 0
     assert s["small"]["device"] == 0 and s["end"]["device"] == 0
     assert s["end"]["events"] == 0 and s["end"]["mallocs"] == s["end"]["frees"]
+
+
+def test_a_pinned_destination_is_copied_to_directly(check):
+    """the link writes pinned memory itself; slots would only add a copy"""
+    s = check("pinned")
+    assert s["pageable"]["chunks"] > 0 and s["pageable"]["direct"] == 0
+    for step in ("pinned", "inside"):
+        assert s[step]["chunks"] == 0 and s[step]["direct"] == 1, step
