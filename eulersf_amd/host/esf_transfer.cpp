@@ -13,9 +13,10 @@
 // ms (1.81 through the slots), 3.2 MB in 0.07 (0.21).
 //
 // The pinned slots belong to the process: at most kStages sets of 16 MB,
-// taken for one copy at a time and freed when the last context goes.  A copy
-// that finds none free, a small one, or one whose threads cannot be started
-// uses hipMemcpyAsync (the last: on one thread).
+// taken for one copy at a time, made once the copies repay it (kRepays) and
+// freed when the last context goes.  A copy that finds none free or a small one
+// uses hipMemcpyAsync; one whose threads cannot be started moves their shares
+// on the calling thread.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -34,16 +35,24 @@ constexpr int kThreads = 8;
 constexpr int kStages = 4;
 // below this a copy is over before the threads are up
 constexpr size_t kLeast = size_t(3) << 20;
+// Bytes of such copies, since there was no context, that go the plain way
+// before a set is pinned for them.  Pinning and freeing one costs 1 to 2 ms and
+// it saves 20 to 55 us a MB: a program with one context at a time and one 22 MB
+// copy of each waited 2.1 ms for it where the plain copy takes 1.25.
+constexpr size_t kRepays = size_t(48) << 20;
 
 struct Stages {
   std::mutex lock;
   int contexts = 0;
+  size_t asked = 0;  // bytes, up to kRepays
   char* mem[kStages] = {};
   bool taken[kStages] = {};
 
-  // a set of 2 kThreads slots, or -1
-  int take() {
+  // a set of 2 kThreads slots for a copy of `bytes`, or -1
+  int take(size_t bytes) {
     std::lock_guard<std::mutex> g(lock);
+    asked = std::min(kRepays, asked + std::min(kRepays, bytes));
+    if (asked < kRepays) return -1;
     for (int i = 0; i < kStages; i++) {
       if (taken[i]) continue;
       if (!mem[i] && hipHostMalloc((void**)&mem[i], 2 * kThreads * kChunk) != hipSuccess) {
@@ -112,7 +121,7 @@ esf_status copyToHost(esf_ctx* ctx, void* dst, const void* src, size_t bytes) {
   const int cpus = (int)std::thread::hardware_concurrency();
   const int threads = std::min<int>(std::min(kThreads, std::max(cpus / 2, 1)),
                                     (int)((bytes + kChunk - 1) / kChunk));
-  const int stage = bytes >= kLeast && threads > 1 && pageable(dst) ? gStages.take() : -1;
+  const int stage = bytes >= kLeast && threads > 1 && pageable(dst) ? gStages.take(bytes) : -1;
   if (stage < 0) {
     ESF_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     ESF_HIP(streamSync(ctx));
@@ -149,6 +158,7 @@ void transferContext(int change) {
   std::lock_guard<std::mutex> g(gStages.lock);
   gStages.contexts += change;
   if (gStages.contexts > 0) return;
+  gStages.asked = 0;
   for (char*& m : gStages.mem) {
     if (m) (void)hipHostFree(m);
     m = nullptr;

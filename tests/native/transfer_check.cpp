@@ -141,5 +141,26 @@ int main(int argc, char** argv) {
     (void)hipHostFree(p);
     esf::transferContext(-1);
   }
+  if (!std::strcmp(what, "pool")) {
+    // one context at a time, one copy each: 20 MB, and 52 at once
+    for (int k = 0; k < 3; k++) {
+      esf::transferContext(1);
+      copy(host.data(), 20 * MB);
+      esf::transferContext(-1);
+    }
+    report("single");
+    esf::transferContext(1);
+    copy(host.data(), dev.size());
+    esf::transferContext(-1);
+    report("big");
+    // a context that goes on: 20 MB four times
+    esf::transferContext(1);
+    for (int k = 0; k < 4; k++) {
+      copy(host.data(), 20 * MB);
+      report(("copy" + std::to_string(k)).c_str());
+    }
+    esf::transferContext(-1);
+    report("end");
+  }
   return 0;
 }

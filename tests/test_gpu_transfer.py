@@ -52,3 +52,16 @@ def test_more_callers_than_slots(esf):
     assert not bad
     for g in scenes:
         g.close()
+
+
+@pytest.mark.parametrize("n", [50, 64, 81])
+def test_downloads_once_slots_are_pinned(esf, n):
+    """past 48 MiB of large copies they go through the slots: whole and partial
+    chunks, and again in a context made after the slots went with the last"""
+    for turn in range(2):
+        g = context(esf, n)
+        v = np.random.default_rng(10 * n + turn).standard_normal(3 * g.nodes)
+        g.upload(esf._abi.F_VELOCITY, v)
+        for _ in range(48 * 2 ** 20 // v.nbytes + 3):
+            np.testing.assert_array_equal(g.download(esf._abi.F_VELOCITY), v)
+        g.close()

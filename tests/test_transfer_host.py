@@ -54,3 +54,14 @@ def test_a_pinned_destination_is_copied_to_directly(check):
     assert s["pageable"]["chunks"] > 0 and s["pageable"]["direct"] == 0
     for step in ("pinned", "inside"):
         assert s[step]["chunks"] == 0 and s[step]["direct"] == 1, step
+
+
+def test_slots_are_pinned_once_the_copies_repay_it(check):
+    """a set is made by the copy that brings the bytes since the first live
+    context to 48 MiB, used from then on, and given back with the last one"""
+    s = check("pool")
+    assert s["single"]["mallocs"] == 0 and s["single"]["direct"] == 3
+    assert s["big"]["chunks"] > 0 and s["big"]["mallocs"] == s["big"]["frees"] == 1
+    for k in range(4):
+        assert (s["copy%d" % k]["chunks"] > 0) == (k >= 2)
+    assert s["end"]["mallocs"] == s["end"]["frees"] == 2
