@@ -1378,7 +1378,9 @@ static esf_status fdSolve(esf_ctx* ctx, double eps, int maxIt, CrScalars* h, int
       a.hostOut = &ctx->hostSc[3];
       if ((st = launchSpmv<double, M_CHECK>(ctx, a))) return st;
       if ((st = waitSlot3(ctx, h))) return st;  // also completes report slot 4
-      if (ctx->hostSc[4].done) break;
+      // (the recursive residual passes a little below eps: the true one may
+      // have passed before)
+      if (h->done || ctx->hostSc[4].done) break;
       chunk = it < 8 ? 1 : 4;
     }
     if (ctx->hostSc[4].done == 1) it = ctx->hostSc[4].iter;

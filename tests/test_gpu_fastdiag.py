@@ -97,3 +97,59 @@ def test_a_grid_past_the_tables_takes_the_refinement(esf):
     it, st, true = solve(esf, (260, 6, 5), [], 1e-8, 4, max_it=100000)
     print(it, true, flush=True)
     assert st == 0 and true < 1e-8
+
+
+class System:
+    """a box with one heavy ball and a right-hand side in S's range; each
+    solve in a context of its own (a context remembers its last count)"""
+
+    def __init__(self, esf, cells, density, seed, scale=1.0):
+        self.esf, self.cells = esf, cells
+        self.text = box_cfg(cells, [{"center": (0.5, 0.5, 0.5), "radius": 0.17,
+                                     "density": density}], eps=1e-10)
+        g = self.context()
+        nx, ny, nz = cells
+        self.minv = g.download(esf._abi.F_MINV).reshape(nz + 1, ny + 1, nx + 1).copy()
+        g.close()
+        for a in range(3):
+            for e in (0, -1):
+                edge = [slice(None)] * 3
+                edge[a] = e
+                self.minv[tuple(edge)] = 0
+        x = np.random.default_rng(seed).standard_normal((nz, ny, nx))
+        self.b = scale * schur(x, self.minv)
+
+    def context(self):
+        g = self.esf.CoupledIntegrator3D.from_cfg_text(self.text, self.esf.ESF_MIXED)
+        g.forces()
+        g.pressureDiag()
+        return g
+
+    def solve(self, eps, max_it, x0=None):
+        """(iterations, starts, reported residual, status, x, x's residual)"""
+        A = self.esf._abi
+        g = self.context()
+        g.upload(A.F_PRESSURE_RHS, self.b.reshape(-1))
+        g.upload(A.F_LAMBDA, np.zeros(self.b.size) if x0 is None else x0.reshape(-1))
+        it, ref, rr, ms, st = g.pressureSolveResident(eps, max_it)
+        x = g.download(A.F_LAMBDA).reshape(self.b.shape)
+        g.close()
+        true = np.linalg.norm(self.b - schur(x, self.minv)) / np.linalg.norm(self.b)
+        return it, ref, rr, st, x, true
+
+
+# (the 2-norm of this system's residual rises from 4 to 5 iterations and is
+# below that of 4 again at 7)
+@pytest.mark.parametrize("k", [4, 7])
+def test_a_passed_check_ends_the_solve(esf, k):
+    """Where the true residual after k iterations lies between 0.95 eps (the
+    recursive residual's test) and eps, the solve ends there and reports that
+    iterate: both residuals are of order 1e-2, off by roundings of 1e-15."""
+    s = System(esf, (24, 27, 22), 1e5, 7)
+    rho = {j: s.solve(1e-30, j)[5] for j in range(4, k + 1)}
+    eps = rho[k] / 0.98
+    print(k, rho, flush=True)
+    assert all(rho[j] > eps for j in range(4, k))  # the check passes at k first
+    it, ref, rr, st, x, true = s.solve(eps, 1000)
+    assert (it, ref, st) == (k, 1, 0)
+    assert abs(rr / true - 1) < 1e-9 and abs(rr / rho[k] - 1) < 1e-9
