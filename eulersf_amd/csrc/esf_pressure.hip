@@ -1411,17 +1411,16 @@ esf_status mixedSolve(esf_ctx* ctx, double eps, int maxIt, int* iters, bool* con
   o.partials = ctx->partials;
   o.first = 1;
   o.hostOut = &ctx->hostSc[3];
-  CrScalars h;
+  CrScalars h{};
   int outer = 0, inner = 0;
   bool residual = true;  // form the residual the refinement starts from
   if (ctx->fd.T) {
     if ((st = fdResidual(ctx, 1, &ctx->hostSc[3]))) return st;
     // where the last solve needed iterations this one's are queued unseen
     // (the wait leaves the device idle for some 20 us); a scene at rest, whose
-    // solves end here, waits instead
-    h.done = 0;
+    // solves end here, waits instead, and so does a solve allowed no iteration
     h.resnorm = std::numeric_limits<double>::infinity();
-    if (ctx->fd.last == 0 && (st = waitSlot3(ctx, &h))) return st;
+    if ((ctx->fd.last == 0 || maxIt < 1) && (st = waitSlot3(ctx, &h))) return st;
     if (!h.done && (st = fdSolve(ctx, eps, maxIt, &h, &inner, &outer))) return st;
     residual = !h.done && inner < maxIt;
   }

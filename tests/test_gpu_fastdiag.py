@@ -153,3 +153,37 @@ def test_a_passed_check_ends_the_solve(esf, k):
     it, ref, rr, st, x, true = s.solve(eps, 1000)
     assert (it, ref, st) == (k, 1, 0)
     assert abs(rr / true - 1) < 1e-9 and abs(rr / rho[k] - 1) < 1e-9
+
+
+def test_no_iterations_allowed(esf):
+    """"cr max iterations" of 0: the start's residual is formed and judged,
+    whether the solve before iterated or not.  From lambda = 0 it is b itself;
+    a lambda solved to 1e-10 passes at 1e-8."""
+    import ctypes
+    from eulersf_amd.cfg import Cfg, params_from_cfg
+    A = esf._abi
+    text = esf.unit_cube_ball_cfg(20, eps=1e-10, max_iterations=2000, velocity=(0.3, -0.5, 0.1))
+
+    def allow(g, most, eps):
+        p = params_from_cfg(Cfg(text=text), 1.0 / 20)
+        p.update(cr_max_iterations=most, divfree_eps=eps, implicit_eps=eps)
+        p = A.Params(**{k: v for k, v in p.items() if k in dict(A.Params._fields_)})
+        p.precision = esf.ESF_MIXED
+        A.check(g.ctx, g.lib.esf_set_params(g.ctx, ctypes.byref(p)))
+
+    g = esf.CoupledIntegrator3D.from_cfg_text(text, esf.ESF_MIXED)
+    g.forces()
+    allow(g, 0, 1e-10)
+    r = g.pcrImplicitSolve()
+    print(r, flush=True)
+    assert r["iterations"][1] == 0 and r["refinements"] == 0 and r["status"] == 1
+    assert r["converged"][1] == 0 and r["rel_residual"][1] == 1.0
+    allow(g, 2000, 1e-10)
+    r = g.pcrImplicitSolve()
+    assert r["status"] == 0 and r["iterations"][1] > 0
+    allow(g, 0, 1e-8)
+    r = g.pcrImplicitSolve()
+    print(r, flush=True)
+    assert r["iterations"][1] == 0 and r["refinements"] == 0
+    assert r["converged"][1] == 1 and r["rel_residual"][1] < 1e-8
+    g.close()
