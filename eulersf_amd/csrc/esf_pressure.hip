@@ -1384,6 +1384,7 @@ static esf_status fdSolve(esf_ctx* ctx, double eps, int maxIt, CrScalars* h, int
       chunk = it < 8 ? 1 : 4;
     }
     if (ctx->hostSc[4].done == 1) it = ctx->hostSc[4].iter;
+    if (it == 0) (*rounds)--;  // queued unseen, and it passed where it stood
     *made += it;
     ctx->fd.last = it;
     if (!(h->resnorm < 0.5 * before)) break;

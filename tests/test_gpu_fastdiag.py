@@ -187,3 +187,20 @@ def test_no_iterations_allowed(esf):
     assert r["iterations"][1] == 0 and r["refinements"] == 0
     assert r["converged"][1] == 1 and r["rel_residual"][1] < 1e-8
     g.close()
+
+
+def test_a_start_that_passes_counts_no_refinement(esf):
+    """the report of a solve that passes where it starts does not depend on
+    what the solve before it took"""
+    s = System(esf, (21, 19, 23), 400.0, 3)
+    A = esf._abi
+    g = s.context()
+    g.upload(A.F_PRESSURE_RHS, s.b.reshape(-1))
+    g.upload(A.F_LAMBDA, np.zeros(s.b.size))
+    it, ref, rr, ms, st = g.pressureSolveResident(1e-10, 1000)
+    assert st == 0 and it > 0 and ref == 1
+    for _ in range(3):
+        it, ref, rr, ms, st = g.pressureSolveResident(1e-9, 1000)
+        print(it, ref, rr, flush=True)
+        assert (st, it, ref) == (0, 0, 0) and rr < 1e-9
+    g.close()
