@@ -363,7 +363,7 @@ ESF_BOUNDS(kFdYX, 256);
 
 // x += alpha p, r -= alpha q, r in FP32 for the preconditioner, |r|^2;
 // alpha = (r . z) / (p . q).  p . q not above 0 (no direction left, or NaN)
-// ends the solve with done = 2.
+// ends the solve with done = 2, x and r as they were.
 template <class GridT>
 __device__ __forceinline__ void kPcgUpdate(const GridT& wg, FdGeom g, long cells,
                                            const double* __restrict__ p,
@@ -376,9 +376,11 @@ __device__ __forceinline__ void kPcgUpdate(const GridT& wg, FdGeom g, long cells
   __shared__ int flag;
   if (blockDone(sc->done, &flag)) return;
   const double pq = blockTotal(nbQ, partsQ, red);
-  const bool ok = pq > 0.0;
-  if (!ok && wg.block() == 0 && threadIdx.x == 0) sc->done = 2;
-  const double alpha = ok ? *rz / pq : 0.0;
+  if (!(pq > 0.0)) {
+    if (wg.block() == 0 && threadIdx.x == 0) sc->done = 2;
+    return;
+  }
+  const double alpha = *rz / pq;
   double rr = 0;
   const long n2 = (cells + 1) >> 1;
   for (long t = wg.block() * (long)blockDim.x + threadIdx.x; t < n2;

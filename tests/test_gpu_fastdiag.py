@@ -204,3 +204,15 @@ def test_a_start_that_passes_counts_no_refinement(esf):
         print(it, ref, rr, flush=True)
         assert (st, it, ref) == (0, 0, 0) and rr < 1e-9
     g.close()
+
+
+def test_no_direction_leaves_x_as_it_was(esf):
+    """a residual past FP32's range has no preconditioned direction (p . q is
+    not a number): the iteration ends the solve and x stays what it was"""
+    s = System(esf, (20, 18, 21), 400.0, 5, scale=1e42)
+    x0 = np.random.default_rng(8).standard_normal(s.b.shape)
+    it, ref, rr, st, x, true = s.solve(1e-10, 1, x0)
+    print(it, ref, rr, st, true, flush=True)
+    assert st == 1
+    np.testing.assert_array_equal(x, x0)
+    assert abs(rr / true - 1) < 1e-9
