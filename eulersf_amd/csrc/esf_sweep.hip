@@ -738,6 +738,10 @@ esf_status computeSdfOn(esf_ctx* ctx, const double* mass, double* phi, int box[6
 constexpr int kScratchDevices = 64;
 std::mutex gScratchLock;
 double* gScratch[kScratchDevices] = {};
+// held by a call while it uses a device's array: tiles of a running sweep wait
+// for words with the epoch they started under, so a second call that reset the
+// tickets and the epoch beneath them would have them wait for good
+std::mutex gScratchUse[kScratchDevices];
 
 // the scratch array's address on device `dev`, looked up with that device
 // current on the first call there
@@ -795,8 +799,12 @@ esf_status esf_compute_sdf_noalloc(esf_ctx* ctx, const double* mass, double* phi
   esf_status st = scratchOn(ctx, ctx->device, &base);
   if (st) return st;
   double* const dm = base + kSdfScratchHead;
-  return computeSdfOn(ctx, mass, phi, box, tight, dm, dm + kSdfScratchNodes, (int*)base,
-                      (unsigned long long*)(dm + 2 * kSdfScratchNodes));
+  std::lock_guard<std::mutex> use(gScratchUse[ctx->device]);
+  st = computeSdfOn(ctx, mass, phi, box, tight, dm, dm + kSdfScratchNodes, (int*)base,
+                    (unsigned long long*)(dm + 2 * kSdfScratchNodes));
+  // (a call that fails may have left sweeps running: they end under the lock)
+  if (st) (void)streamSync(ctx);
+  return st;
 }
 
 esf_status esf_extend_vector_field(esf_ctx* ctx, const int box[6], const double* mass,

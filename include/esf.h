@@ -263,9 +263,8 @@ esf_status esf_compute_sdf(esf_ctx* ctx, const double* mass, double* phi, int bo
  * counters live in a static device array of the library, one per GPU, held
  * while the process lives: 45.5 MB, enough for grids of at most 129^3 =
  * 2,146,689 nodes (larger grids: ESF_ERR_INVALID).  Every call on a GPU
- * uses that GPU's one array, so calls that overlap on one GPU (from
- * several threads or contexts) race; calls in sequence are safe, each
- * starts its counters afresh. */
+ * uses that GPU's one array, for itself while it runs: calls from several
+ * threads or contexts take their turns, each starts its counters afresh. */
 esf_status esf_compute_sdf_noalloc(esf_ctx* ctx, const double* mass, double* phi,
                                    int box[6], int tight[6]);
 /* DEFOR_SOLID_3D::extendVectorField (DEFOR_SOLID_3D.cpp:566-574): four

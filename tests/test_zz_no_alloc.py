@@ -55,3 +55,36 @@ def test_noalloc_sdf_refuses_a_grid_beyond_its_scratch(esf):
     assert st == _abi.ESF_ERR_INVALID
     assert b"scratch" in g.lib.esf_last_error(g.ctx)
     g.close()
+
+
+def test_noalloc_sdf_calls_from_several_threads_take_turns(esf):
+    """the calls share one array per GPU: started together from contexts of
+    their own they give what they give alone, bitwise"""
+    import threading
+    sizes = (24, 32, 40)
+    scenes, masses, want = [], [], []
+    for k, n in enumerate(sizes):
+        g = esf.CoupledIntegrator3D.from_cfg_text(esf.unit_cube_ball_cfg(n))
+        m = ball_mass(n, (0.5, 0.45 + 0.05 * k, 0.5), 0.2)
+        scenes.append(g)
+        masses.append(m)
+        want.append(g.computeSDF(m))
+    start = threading.Barrier(len(sizes))
+    bad = []
+
+    def run(k):
+        start.wait(30)
+        for _ in range(4):
+            phi, box, tight = scenes[k].computeSDFNoAlloc(masses[k])
+            if not (np.array_equal(phi.view(np.int64), want[k][0].view(np.int64)) and
+                    list(box) == list(want[k][1]) and list(tight) == list(want[k][2])):
+                bad.append(k)
+
+    team = [threading.Thread(target=run, args=(k,)) for k in range(len(sizes))]
+    for t in team:
+        t.start()
+    for t in team:
+        t.join()
+    assert not bad
+    for g in scenes:
+        g.close()
