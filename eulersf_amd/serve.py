@@ -120,6 +120,15 @@ class BatchRunner:
         self.scenes = []
 
 
+def note_bytes(server, rec, g):
+    """what a context holds, into its record and the server's admission
+    estimate (the caller holds the server's lock): once it is made and again
+    after its first step, which brings scratch sized by the solids' boxes"""
+    rec["bytes"] = g.device_bytes()
+    server.bytes_per_node = max(server.bytes_per_node,
+                                rec["bytes"] / float((rec["n"] + 1) ** 3))
+
+
 class Server:
     """Continuous batching of scene requests.  A request (arrival time, N,
     K steps, cfg text) is admitted when fewer than `max_active` scenes are
@@ -164,11 +173,12 @@ class Server:
             g = None
             try:
                 g = CoupledIntegrator3D.from_cfg_text(req["text"], self.precision)
-                rec["bytes"] = g.device_bytes()
                 with self.lock:
-                    self.bytes_per_node = max(self.bytes_per_node,
-                                              rec["bytes"] / float((req["n"] + 1) ** 3))
-                step_scene(g, req["k"], rec["lat"])
+                    note_bytes(self, rec, g)
+                step_scene(g, min(1, req["k"]), rec["lat"])
+                with self.lock:
+                    note_bytes(self, rec, g)
+                step_scene(g, req["k"] - 1, rec["lat"])
                 if self.on_done is not None:
                     self.on_done(req, g)
             except Exception as e:  # kept in the record, reported by the caller
@@ -274,13 +284,12 @@ class BatchedServer:
                 g = None
                 try:
                     g = CoupledIntegrator3D.from_cfg_text(req["text"], self.precision)
-                    rec["bytes"] = g.device_bytes()
+                    with cv:
+                        note_bytes(self, rec, g)
                 except Exception as e:  # kept in the record, reported by the caller
                     rec["error"] = repr(e)
                 with cv:
                     if rec["error"] is None:
-                        self.bytes_per_node = max(self.bytes_per_node,
-                                                  rec["bytes"] / float((req["n"] + 1) ** 3))
                         ready[self.lane_of(req["n"])].append([rec, g, est, 0])
                     else:
                         rec["end"] = time.perf_counter() - t_start
@@ -315,6 +324,9 @@ class BatchedServer:
                     a[3] += 1
                     if err is not None:
                         rec["error"] = err
+                    elif a[3] == 1:
+                        with cv:
+                            note_bytes(self, rec, g)
                     if a[3] >= rec["k"] or err is not None:
                         if self.on_done is not None and err is None:
                             self.on_done({"id": rec["id"], "n": rec["n"], "k": rec["k"]}, g)

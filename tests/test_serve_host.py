@@ -1,8 +1,10 @@
 """Host logic of the batched / served workloads (no GPU): request streams
 and scene generation."""
 import numpy as np
+import pytest
 
-from eulersf_amd.serve import poisson_requests, random_scene, summarize
+from eulersf_amd import serve
+from eulersf_amd.serve import BatchedServer, Server, poisson_requests, random_scene, summarize
 
 
 def test_poisson_stream_statistics():
@@ -36,3 +38,38 @@ def test_summary_of_records():
     assert s["steps"] == 3 and s["steps_per_s"] == 3.0
     assert s["cells_steps_per_s"] == 2 * 32 ** 3 + 64 ** 3
     assert s["completion_latency_ms"]["p50"] == 600.0
+
+
+class GrowingScene:
+    """a context that holds 1300 bytes per node once made and 1500 once it
+    has stepped (the sweeps' scratch comes with a FLIP scene's first step)"""
+
+    def __init__(self, n):
+        self.nodes, self.stepped = (n + 1) ** 3, False
+
+    @classmethod
+    def from_cfg_text(cls, text, precision):
+        return cls(int(text))
+
+    def device_bytes(self):
+        return (1500 if self.stepped else 1300) * self.nodes
+
+    def stepImplicit(self, alpha):
+        self.stepped = True
+        return {"status": 0}
+
+    def close(self):
+        pass
+
+
+@pytest.mark.parametrize("kind", [Server, BatchedServer])
+def test_admission_sees_what_contexts_hold_once_they_step(monkeypatch, kind):
+    monkeypatch.setattr(serve, "CoupledIntegrator3D", GrowingScene)
+    monkeypatch.setattr(serve, "step_batch", lambda gs: [g.stepImplicit(-1.0) for g in gs])
+    reqs = [{"id": i, "t": 0.0, "n": 40 + i, "k": 1 + 2 * i, "text": str(40 + i)} for i in range(3)]
+    s = kind(1 << 40, 4)
+    recs, makespan, info = s.run(reqs)
+    assert sorted(r["id"] for r in recs) == [0, 1, 2] and all(r["error"] is None for r in recs)
+    for r in recs:
+        assert len(r["lat"]) == r["k"] and r["bytes"] == 1500 * (r["n"] + 1) ** 3
+    assert s.bytes_per_node == pytest.approx(1500.0)
