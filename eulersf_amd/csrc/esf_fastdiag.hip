@@ -18,10 +18,11 @@
 // modes), which S shares whatever the masses.  For every x,
 // x^T S x / x^T S0 x lies between the smallest and the largest 1 / m, so the
 // iteration count depends on the spread of the node masses only, not on the
-// grid: 4 iterations to 1e-12 where solid and fluid weigh the same, about 15
-// at a density ratio of 2, 57 at 100, where Jacobi-preconditioned CR needs
-// some thousands (the near-checkerboard modes make S's condition number
-// grow as n^4).
+// grid.  Measured to 1e-12, one ball in a box of 24^3 to 64^3: 3 iterations
+// where solid and fluid weigh the same, 15 at a density ratio of 2, 37 at 10,
+// 95-101 at 100, 150-182 at 1000, where Jacobi-preconditioned CR needs some
+// thousands (the near-checkerboard modes make S's condition number grow as
+// n^4).
 //
 // One application is six dense products along an axis; they run on the
 // matrix cores (FP32 16x16x4) in three kernels: x and y forward, z forward

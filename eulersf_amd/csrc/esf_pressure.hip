@@ -1350,8 +1350,11 @@ static esf_status fdResidual(esf_ctx* ctx, int first, CrScalars* hostOut) {
 // halve the residual; lambda then holds the last iterate.
 static esf_status fdSolve(esf_ctx* ctx, double eps, int maxIt, CrScalars* h, int* made,
                           int* rounds) {
-  // past 200 iterations the node masses spread over more than three
-  // decades, and the Jacobi scaling of the FP32 CR takes them better
+  // A bound on what a solve that does not fall can waste.  Balls of a thousand
+  // times the fluid's density take 150-184 iterations to 1e-12 on 24^3, 48^3
+  // and 64^3 grids, 1e4 to 1e6 times 211-280 if left to run, where the FP32 CR
+  // alone takes 1400-7700 of its own (4-9 ms against 20-113); handed over at
+  // 200 they end in 5-9.5 ms, some a fifth sooner and some a third later.
   constexpr int kFdIterations = 200;
   const int most = std::min(maxIt, kFdIterations);
   esf_status st;

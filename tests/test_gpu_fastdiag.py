@@ -216,3 +216,45 @@ def test_no_direction_leaves_x_as_it_was(esf):
     assert st == 1
     np.testing.assert_array_equal(x, x0)
     assert abs(rr / true - 1) < 1e-9
+
+
+# Residuals are formed twice, on the device and here: each is off by roundings
+# of b and S x, some 20 terms of at most |b| (S's rows scale with b's), so by
+# less than 20 2^-53 = 2.3e-15 of |b| each.
+ROUNDING = 5e-15
+
+
+def test_hands_over_to_the_refinement_past_its_limit(esf):
+    """a ball a million times the fluid's density needs more than 200
+    preconditioned iterations to 1e-12: the refinement goes on from there and
+    ends at the true residual"""
+    s = System(esf, (24, 24, 24), 1e9, 1)
+    it, ref, rr, st, x, true = s.solve(1e-12, 60000)
+    print(it, ref, rr, true, flush=True)
+    assert st == 0 and it > 200 and ref >= 2
+    assert rr < 1e-12 and abs(rr - true) < ROUNDING
+
+
+@pytest.mark.parametrize("density, max_it", [(1e5, 1), (1e5, 3), (1e5, 30), (1e9, 199), (1e9, 200),
+                                             (1e9, 201), (1e9, 230)])
+def test_a_limit_before_convergence(esf, density, max_it):
+    """the iteration limit short of convergence, inside the preconditioned
+    iterations and past their hand-over: not converged, no iteration past the
+    limit, and the residual reported is that of the x returned"""
+    s = System(esf, (24, 27, 22), density, 2)
+    it, ref, rr, st, x, true = s.solve(1e-13, max_it)
+    print(density, max_it, it, ref, rr, true, flush=True)
+    assert st == 1 and it <= max_it
+    assert it == max_it or max_it > 200
+    assert abs(rr - true) < 1e-9 * true + ROUNDING
+
+
+def test_a_restart_that_does_not_fall_hands_over(esf):
+    """a tolerance below the rounding of the residual itself: the recursive
+    residual passes, the true one stays above, the restart does not halve it and
+    the refinement (the third start) is left with the rest"""
+    s = System(esf, (24, 27, 22), 400.0, 4)
+    it, ref, rr, st, x, true = s.solve(1e-16, 60)
+    print(it, ref, rr, true, flush=True)
+    assert st == 1 and ref >= 3 and it == 60
+    assert abs(rr - true) < ROUNDING and true < 10 * ROUNDING
