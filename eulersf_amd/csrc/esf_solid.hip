@@ -341,10 +341,12 @@ __device__ __forceinline__ void kSolidCell(const GridT& wg, Dims d, CellBodies<N
                                            const double* __restrict__ xin, const CrScalars* sc,
                                            SolidPartials sp) {
 #pragma clang fp contract(on)
-  int body = 0;
-  for (int b = 1; b < bodies.n; b++)
-    if (wg.block() >= bodies.b[b].start) body = b;
-  const CellBody& cb = bodies.b[body];
+  // (selected entry by entry: an index known only here would have the whole
+  // table copied to private memory in a batched launch)
+  CellBody cb = bodies.b[0];
+#pragma unroll
+  for (int b = 1; b < NB; b++)
+    if (b < bodies.n && wg.block() >= bodies.b[b].start) cb = bodies.b[b];
   const int nValid = cb.nValid, cap = cb.cap;
   const int* __restrict__ cornerDof = cb.cornerDof;
   const double* __restrict__ cellMat = cb.cellMat;
@@ -779,6 +781,11 @@ static void cellPass(esf_ctx* ctx, const double* in, const CrScalars* sc,
     pass(std::integral_constant<int, 2>{});
 }
 
+// The node pass's blocks are the partial sums of the solve, so their size goes
+// by the scene alone, also in a batched step (its results are bitwise the
+// scene's own); scenes on either side of kSpreadLanes then launch apart.  64
+// scenes of 32^3 to 96^3: 12 launches of kSolidNode<0> of 54 us where one size
+// took 6 of 99 us.
 static int nodeThreads(const esf_ctx* ctx) {
   return 3L * ctx->nSolid < kSpreadLanes ? 128 : kNodeThreads;
 }
