@@ -912,8 +912,9 @@ static esf_status launchFlat(esf_ctx* ctx, int nb, const SpmvArgs<double>& a) {
   else
     launchTimed<ESF_KT(kSpmvFlat, MODE, 256)>(ctx, cls, dim3(blocks), dim3(256), d, a,
                                               cdiv(d.CX, FX), cdiv(d.CY, FY));
-  if (hipGetLastError() == hipSuccess) return ESF_OK;
-  ctx->err = "kSpmvFlat launch";
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return ESF_OK;
+  ctx->err = std::string("kSpmvFlat launch: ") + hipGetErrorString(e);
   return ESF_ERR_DEVICE;
 }
 

@@ -101,3 +101,19 @@ def test_a_start_that_passes_is_returned_unchanged(esf, monkeypatch):
         assert st2 == 0 and it2 == 0 and rr2 < 1e-9
         np.testing.assert_array_equal(x2.view(np.int64), x.view(np.int64))
     g.close()
+
+
+@pytest.mark.parametrize("cells", [(16, 8, 4), (129, 64, 64)])
+def test_a_refused_launch_says_why(esf, cells):
+    """a runtime error found at a launch (here one left by an allocation that
+    no device can grant) is named, by the small-grid operator and the march"""
+    import ctypes
+    g = esf.CoupledIntegrator3D.from_cfg_text(box_cfg(cells, []))
+    g.forces()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    p = ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(1 << 60)) != 0
+    with pytest.raises(esf._abi.EsfError, match="launch: out of memory"):
+        g.getMatVecMult(np.zeros(g.cells))
+    assert not g.getMatVecMult(np.zeros(g.cells)).any()
+    g.close()
